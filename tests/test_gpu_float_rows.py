@@ -208,3 +208,30 @@ def test_wide_rows_past_64k_of_lds(oracle, quant, ffn):
         assert tg == oracle.argmax(gpu.logits) and d < F32_TOL, (pos, d)
     gpu.close()
     ref.close()
+
+
+@pytest.mark.parametrize("quant", [L.QUANT_F32, L.QUANT_F16])
+@pytest.mark.parametrize("hidden,inter,heads,kv,d,vocab", [
+    (64, 96, 1, 1, 64, 33),         # rows shorter than a wave's 64 words, 1-wave workgroups, fewer rows than CUs
+    (264 * 4, 1536, 9, 3, 64, 301),  # a ragged last word group (264 / 132 words), 6-wave workgroups
+    (2080, 4160, 16, 4, 128, 2055),  # 8-wave workgroups: several rows per wave, uneven blocks of rows
+])
+def test_float_rows_grid_edges_match_the_oracle(oracle, quant, hidden, inter, heads, kv, d, vocab):
+    """The float-row GEMV's grids and row ends: two layers, three positions, within the fp32-accumulation bar."""
+    seed, layers = 7, 2
+    dims = dict(vocab_size=vocab, hidden_dim=hidden, intermediate_dim=inter, num_layers=layers, num_heads=heads,
+                num_kv_heads=kv, head_dim=d, rms_norm_eps=1e-5, rope_theta=10000.0, qkv_bias=1, tied_lm_head=1)
+    gpu = HipDecodeEngine(dict(dims, quant_mode=quant), seed=seed, norm_sigma=0.1, max_seq_len=16)
+    ref = oracle.Engine(dict(dims, max_seq_len=16), seed=seed, sigma=0.02, norm_sigma=0.1, q4_0=False, kv_bf16=True,
+                        w_f16=quant == L.QUANT_F16, threads=8)
+    for pos, tok in enumerate(oracle.prompt_tokens(seed, 3, vocab)):
+        tg = gpu.forward_step(int(tok), pos)
+        rows = [_device_kv(gpu.arena, layer, kv, 16, d, pos + 1) for layer in range(layers)]
+        for layer in range(layers):
+            kr, vr = ref.kv_cache(layer)
+            kr[:pos], vr[:pos] = rows[layer][0][:pos], rows[layer][1][:pos]
+        ref.forward_forced(int(tok), pos, np.stack([r[0][pos] for r in rows]), np.stack([r[1][pos] for r in rows]))
+        err = float(np.max(np.abs(gpu.logits - ref.logits)))
+        assert tg == oracle.argmax(gpu.logits) and err < F32_TOL, (pos, err)
+    gpu.close()
+    ref.close()

@@ -341,8 +341,10 @@ int vx_record_error(hipError_t e);  // vx_host.cpp: the first error of a step, r
 enum { VX_EPI_STORE = 0, VX_EPI_RESID = 1, VX_EPI_SWIGLU = 2, VX_EPI_ARGMAX = 3 };
 hipError_t vx_launch_gemv(const VxMat& m, const VxGemvArgs& a, int epi, uint32_t max_wgs, hipStream_t st);
 // The float-row GEMV (vx_gemv_f.hip) that vx_launch_gemv runs for VX_FMT_F32 / VX_FMT_F16 matrices,
-// on `wgs` workgroups (vx_gemv_grid of the matrix's tiles).
-hipError_t vx_launch_gemv_f(const VxMat& m, const VxGemvArgs& a, int epi, uint32_t wgs, hipStream_t st);
+// its grid from the rows (past 8192 rows at most max_wgs workgroups; the LM head: head_wgs, vx_gemv_grid
+// of the matrix's tiles).
+hipError_t vx_launch_gemv_f(const VxMat& m, const VxGemvArgs& a, int epi, uint32_t head_wgs, uint32_t max_wgs,
+                            hipStream_t st);
 hipError_t vx_launch_attention(const VxAttnArgs& a, uint32_t d, hipStream_t st);
 // vx_qkv_attn.hip: whether matrix m (the fused [q; k; v] rows) and the head shape take the fused
 // QKV + attention launch; the launch with p GEMV workgroups per KV head; and the device check that

@@ -784,7 +784,7 @@ hipError_t vx_launch_gemv(const VxMat& m, const VxGemvArgs& a, int epi, uint32_t
         case VX_FMT_Q4: return vx_launch_gemv_tiled<VX_FMT_Q4>(m, a, epi, max_wgs, st);
         case VX_FMT_G64: return vx_launch_gemv_g64(m, a, epi, max_wgs, st);
         case VX_FMT_F32:
-        case VX_FMT_F16: return vx_launch_gemv_f(m, a, epi, vx_gemv_wgs(m.n_tiles, max_wgs), st);
+        case VX_FMT_F16: return vx_launch_gemv_f(m, a, epi, vx_gemv_wgs(m.n_tiles, max_wgs), max_wgs, st);
         default: return hipErrorInvalidValue;
     }
 }

@@ -174,3 +174,17 @@ def test_mla_bad_arguments():
     m = C.c_void_p()
     assert lib.velox_hip_mla_create(C.byref(c), C.byref(m)) == L.ESHAPE
     assert lib.velox_hip_mla_builtin_config(b"nope", 64, 1, C.byref(L.MlaConfig())) == L.EINVAL
+
+
+@pytest.mark.parametrize("heads,batch,splits,max_seq", [
+    (64, 16, 16, 96),    # splits of one 32-position chunk, most of them empty
+    (64, 32, 8, 1300),   # splits of up to six chunks, sequences ending anywhere in them
+    (128, 5, 28, 700),   # two head groups, 280 workgroups dealt unevenly to the eight XCDs
+])
+def test_mla_attention_64_heads_vs_oracle(oracle, heads, batch, splits, max_seq):
+    """The 64-head attention workgroups at the edges of chunks and splits: contexts of 0 positions, one
+    less and one more than whole 32-position chunks, and the longest."""
+    cfg = dict(SMALL, num_heads=heads, kv_lora_rank=512)
+    edges = [0, 1, 31, 32, 33, 63, 64, 65, 94, max_seq - 1, max_seq // 2, max_seq // 3, 95]
+    ctxs = [min(edges[b % len(edges)] + (b // len(edges)) * 7, max_seq - 1) for b in range(batch)]
+    _check_layer(oracle, cfg, batch=batch, ctxs=ctxs, steps=1, max_seq=max_seq, splits=splits)

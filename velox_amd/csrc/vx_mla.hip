@@ -1026,6 +1026,316 @@ __global__ __launch_bounds__(64 * W * LS, 1) void vx_mla_attn_kernel(VxMlaAttnAr
     }
 }
 
+// The attention of 64 heads of one (split, sequence), where a grid of such workgroups fills the chip.
+// The kernel above spent most of a 32-position chunk (2.8 us of 1.1k matrix-core clocks) between its
+// three barriers: registers -> LDS staging, partial scores through LDS, every wave of a head pair running
+// the same softmax, and the pair's P.V reading half the chunk per 16 heads. Here:
+// * the chunks come in by direct-to-LDS loads, four buffers, requested three chunks ahead. A row's
+//   16-byte blocks lie XOR-swizzled by the row's low three bits (the lane that loads a block picks it),
+//   so neither the scores' row reads nor P.V's transposed reads meet in a bank beyond the two passes
+//   their bytes need;
+// * scores: wave (hm, pb) computes S^T of positions 16 pb .. + 15 for heads 16 hm .. + 15 over all
+//   LR + DR dimensions (its q operands stay in registers), so no partial sums; the two waves of a head
+//   tile exchange their maxima and each exponentiates its own 16 positions once;
+// * P.V: wave w accumulates all 64 heads over LR / 8 dimensions, so each latent value is read once per
+//   workgroup (P, 4 KiB, once per wave);
+// * P.V of chunk i runs in the phase of the scores of chunk i + 1: two barriers per chunk.
+// * O leaves through LDS as whole lines, and a sequence's workgroups share an XCD (below).
+// DeepSeek-V3 at B = 16, 8 splits of 17 chunks: 47.4 -> 36.0 us (kernel trace); what is left is about 13 us
+// before the first chunk and after the last (q, the partials' 16.8 MB) and 1.4 us per chunk, of which
+// barriers and softmax 0.5, the scores' LDS reads 0.3, P.V 0.3, the loads 0.2 (by elimination).
+template <int N>
+__device__ __forceinline__ void vm_wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+__device__ __forceinline__ void vm_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// 16 bytes per lane from base + off (off per lane) to the 1 KiB of LDS at byte offset lds (both uniform)
+__device__ __forceinline__ void vm_dma16(const void* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+
+// The maximum over the four 16-lane groups, in every lane (lane swaps: no LDS round trip).
+__device__ __forceinline__ float vm_max_groups(float v) {
+    const uint32_t a = __float_as_uint(v);
+    const auto p = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+    const uint32_t m = __float_as_uint(fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1])));
+    const auto q = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+
+template <int LR, int DR>
+constexpr size_t vx_mla_attn64_lds() {  // four chunks, P, alpha, the waves' maxima
+    return (size_t)4 * 32 * (LR + DR) * 2 + 64 * 32 * 2 + 64 * 4 + 2 * 64 * 4;
+}
+
+template <int LR, int DR>
+__global__ __launch_bounds__(512) void vx_mla_attn64_kernel(VxMlaAttnArgs a, uint32_t batch) {
+    if ((a.active_mask & 1ULL) == 0ULL) return;
+    constexpr int R = LR + DR, NCK = R / 32, RB = R / 8;        // 32-dimension steps, 16-byte blocks per row
+    constexpr uint32_t kBuf = 32u * R * 2u, kUnits = kBuf / 1024u;  // bytes and 1 KiB units of a chunk
+    constexpr uint32_t UW = (kUnits + 7u) / 8u;                 // units per wave, at most
+    static_assert(LR == 512 && R % 64 == 0 && kBuf % 1024u == 0, "8 waves of 64 dimensions; whole swizzle groups and units");
+    extern __shared__ __align__(16) unsigned char vm_smem[];
+    uint16_t* p_s = (uint16_t*)(vm_smem + 4u * kBuf);  // [64 heads][32]: element e of lane group g at 8 g + e
+    float* alpha_s = (float*)(p_s + 64 * 32);          // [64]
+    float* pm_s = alpha_s + 64;                        // [2][64]: maxima, at the end the sums l
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int hm = wave >> 1, pb = wave & 1;
+    const int col = lane & 15, grp = lane >> 4;
+    // The dispatcher deals workgroup i to XCD i % 8: XCD x takes items [x share, (x + 1) share) in the order
+    // (sequence, split, head group), so a split's head groups read its latent rows, and a sequence's splits
+    // its q, through one L2 (q through all eight cost about 4 us of a launch).
+    const uint32_t zg = a.nh / 64u, items = batch * a.splits * zg, share = gridDim.x / 8u;
+    const uint32_t item = (blockIdx.x & 7u) * share + (blockIdx.x >> 3);
+    if (item >= items) return;  // the grid is rounded up to whole shares
+    const uint32_t sp = item / zg % a.splits, b = item / (zg * a.splits), hbase = item % zg * 64u;
+    const uint32_t head = hbase + 16u * (uint32_t)hm + (uint32_t)col;
+    const uint64_t step = a.states[b].step;
+    const uint32_t pos = __builtin_amdgcn_readfirstlane(step < (uint64_t)a.s_max ? (uint32_t)step : a.s_max - 1u);
+    const uint32_t len = pos + 1u;
+    const uint32_t chunk = ((a.s_max + a.splits - 1u) / a.splits + 31u) & ~31u;
+    const uint32_t t0 = sp * chunk, t1 = min(len, t0 + chunk);
+    const uint32_t n = t1 > t0 ? (t1 - t0 + 31u) >> 5 : 0u;
+    const uint16_t* t0_base = a.cache + (size_t)b * a.cache_bstride + (size_t)t0 * R;  // (t0 may pass pos: not read then)
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)vm_smem;
+
+    // ---- chunk j into buffer j % 4: unit u = wave + 8 i, lane l fills 16-byte slot 64 u + l = (row, sb)
+    // with block sb ^ (row & 7) of that row (rows past pos: row pos again, masked below) ----
+    uint32_t urow[UW], ublk[UW];
+#pragma unroll
+    for (uint32_t i = 0; i < UW; ++i) {
+        const uint32_t s16 = min(64u * ((uint32_t)wave + 8u * i) + (uint32_t)lane, 32u * RB - 1u);
+        urow[i] = s16 / RB;
+        ublk[i] = 16u * ((s16 % RB) ^ (urow[i] & 7u));
+    }
+    const bool full = (uint32_t)wave + 8u * (UW - 1u) < kUnits;  // this wave fills UW units, else UW - 1
+    auto dma = [&](uint32_t j) {
+#pragma unroll
+        for (uint32_t i = 0; i < UW; ++i)
+            if (i + 1u < UW || full)
+                vm_dma16(t0_base, min(32u * j + urow[i], pos - t0) * (uint32_t)(2 * R) + ublk[i],
+                         lds0 + (j & 3u) * kBuf + ((uint32_t)wave + 8u * i) * 1024u);
+    };
+    if (n) {
+        dma(0u);
+        if (n > 1u) dma(1u);
+    }
+
+    // ---- q operands of head col (as in the kernel above): scaled, the RoPE part rotated, bf16. The two
+    // waves of a head tile load every other 32-dimension step each and pass them on through buffers 2, 3 ----
+    vm_b8 qreg[NCK];
+    {
+        const float* qa = a.qabs + ((size_t)b * a.nh + head) * LR + 32 * pb + 8 * grp;
+        vm_b8* qx = (vm_b8*)(vm_smem + 2u * kBuf) + (size_t)wave * (NCK / 2) * 64 + lane;
+        static_assert(8u * (NCK / 2) * 1024u <= 2u * kBuf, "the exchange fits two buffers");
+        float4 x[LR / 64][2];
+#pragma unroll
+        for (int c = 0; c < LR / 64; ++c) {
+            x[c][0] = *(const float4*)(qa + 64 * c);
+            x[c][1] = *(const float4*)(qa + 64 * c + 4);
+        }
+        // the RoPE part: step pb holds the first (x1) or second (x2) halves of the 32 pairs
+        const float* qr = a.q32 + (size_t)b * a.nh * a.dq + (size_t)head * a.dq + a.dn + 8 * grp;
+        const float2* rp = a.rope + (size_t)pos * (DR / 2) + 8 * grp;
+        float4 r1[2], r2[2], cs[4];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            r1[e] = *(const float4*)(qr + 4 * e);
+            r2[e] = *(const float4*)(qr + DR / 2 + 4 * e);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cs[e] = *(const float4*)(rp + 2 * e);
+#pragma unroll
+        for (int c = 0; c < NCK / 2; ++c) {
+            float v[8];
+            if (c < LR / 64) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = ((const float*)x[c])[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float2 o = vm_rope_pair(((const float*)r1)[e], ((const float*)r2)[e], ((const float2*)cs)[e]);
+                    v[e] = pb ? o.y : o.x;
+                }
+            }
+            vm_b8 q;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) q[e] = (__bf16)(v[e] * a.qscale);
+            qx[c * 64] = q;
+        }
+        vm_barrier();
+        const vm_b8* q0 = (const vm_b8*)(vm_smem + 2u * kBuf) + (size_t)(wave & ~1) * (NCK / 2) * 64 + lane;
+#pragma unroll
+        for (int c = 0; c < NCK; ++c) qreg[c] = q0[((c & 1) * (NCK / 2) + c / 2) * 64];
+        vm_barrier();
+    }
+    if (n > 2u) dma(2u);
+
+    float m_run = -INFINITY, l_run = 0.0f;
+    vm_f4 o_acc[4][4];  // [head tile][16 dimensions of this wave's 64]: dimensions 4 grp + i of head col
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) o_acc[h][nt] = vm_f4{0.f, 0.f, 0.f, 0.f};
+
+    // byte offsets in a chunk: the scores' block 4 c + grp of row 16 pb + col (c even / odd), and P.V's
+    // 8 bytes of row 4 grp + col / 4, dimensions 64 wave + 16 nt + 4 (col % 4)
+    const uint32_t krow = 16u * (uint32_t)pb + (uint32_t)col;
+    uint32_t koff[2], voff[4];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) koff[e] = krow * (2u * R) + 16u * ((4u * (uint32_t)e + (uint32_t)grp) ^ (krow & 7u));
+    const uint32_t vrow = 4u * (uint32_t)grp + ((uint32_t)col >> 2);
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+        voff[nt] = vrow * (2u * R) + 128u * (uint32_t)wave +
+                   16u * ((2u * (uint32_t)nt + (((uint32_t)col & 3u) >> 1)) ^ (vrow & 7u)) + 8u * ((uint32_t)col & 1u);
+
+    vm_f4 sc = vm_f4{0.f, 0.f, 0.f, 0.f};
+    float mx = -INFINITY;
+    // scores of chunk j: sc[i] = S[position 16 pb + 4 grp + i][head col], positions past the split masked;
+    // the tile's maximum per head to LDS
+    auto scores = [&](uint32_t j) {
+        const unsigned char* kb = vm_smem + (j & 3u) * kBuf;
+        // two chains, so that one product's latency passes behind the other's
+        vm_f4 s0 = vm_f4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+        for (int c = 0; c < NCK; c += 2) {
+            const vm_b8 k0 = *(const vm_b8*)(kb + koff[0] + 64u * (uint32_t)c);
+            const vm_b8 k1 = *(const vm_b8*)(kb + koff[1] + 64u * (uint32_t)c);
+            s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qreg[c], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qreg[c + 1], s1, 0, 0, 0);
+        }
+        sc = s0 + s1;
+        mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t p = t0 + 32u * j + 16u * (uint32_t)pb + 4u * (uint32_t)grp + (uint32_t)i;
+            sc[i] = p < t1 ? sc[i] : -INFINITY;
+            mx = fmaxf(mx, sc[i]);
+        }
+        mx = vm_max_groups(mx);
+        if (lane < 16) pm_s[64 * pb + 16 * hm + lane] = mx;
+    };
+    // the chunk's probabilities against the (lazy) running maximum, to LDS; alpha rescales the sums
+    auto probs = [&]() {
+        mx = fmaxf(mx, pm_s[64 * (1 - pb) + 16 * hm + col]);
+        const float m_new = (m_run == -INFINITY || mx > m_run + kMlaLazy) ? mx : m_run;
+        const float alpha = m_run == -INFINITY ? 1.0f : vm_exp2(m_run - m_new);  // (before it: zero sums)
+        float lt = 0.0f;
+        uint16_t pq[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float p = sc[i] == -INFINITY ? 0.0f : vm_exp2(sc[i] - m_new);
+            lt += p;
+            pq[i] = __builtin_bit_cast(uint16_t, (__bf16)p);
+        }
+        l_run = l_run * alpha + lt;
+        m_run = m_new;
+        *(uint2*)(p_s + (16 * hm + col) * 32 + 8 * grp + 4 * pb) =
+            make_uint2(pq[0] | ((uint32_t)pq[1] << 16), pq[2] | ((uint32_t)pq[3] << 16));
+        if (pb == 0 && lane < 16) alpha_s[16 * hm + lane] = alpha;
+    };
+    // O += P V over the chunk's 32 positions (k-elements e < 4: position 4 grp + e, e >= 4: 16 + 4 grp + e - 4)
+    auto pv = [&](uint32_t j) {
+        const unsigned char* kb = vm_smem + (j & 3u) * kBuf;
+        float al[4];
+        bool grew = false;
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            al[h] = alpha_s[16 * h + col];
+            grew |= al[h] != 1.0f;
+        }
+        vm_b8 pop[4], vop[4];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) pop[h] = *(const vm_b8*)(p_s + (16 * h + col) * 32 + 8 * grp);
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            const vm_s4 lo = vm_lds_tr4((const __bf16*)(kb + voff[nt]));
+            const vm_s4 hi = vm_lds_tr4((const __bf16*)(kb + voff[nt] + 16u * 2u * R));
+            vop[nt] = __builtin_bit_cast(vm_b8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+        if (__any(grew)) {  // wave-uniform
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+#pragma unroll
+                for (int nt = 0; nt < 4; ++nt) o_acc[h][nt] *= al[h];
+        }
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+                o_acc[h][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop[nt], pop[h], o_acc[h][nt], 0, 0, 0);
+    };
+    // chunk j has landed in every wave's share: at most `newer` chunks requested after it are outstanding
+    auto wait_chunk = [&](uint32_t newer) {
+        constexpr int F = (int)UW;
+        if (newer >= 2u) { if (full) vm_wait_vm<2 * F>(); else vm_wait_vm<2 * (F - 1)>(); }
+        else if (newer == 1u) { if (full) vm_wait_vm<F>(); else vm_wait_vm<F - 1>(); }
+        else vm_wait_vm<0>();
+    };
+
+    if (n) {
+        wait_chunk(n - 1u);
+        vm_barrier();
+        scores(0u);
+        vm_barrier();
+        probs();
+        wait_chunk(n > 2u ? 1u : 0u);  // chunk 1 (chunks 1 and 2 requested)
+        vm_barrier();
+        for (uint32_t i = 0; i + 1u < n; ++i) {
+            // buffer (i + 3) % 4 held chunk i - 1, whose last reads the barrier above follows
+            if (i + 3u < n) dma(i + 3u);
+            scores(i + 1u);
+            pv(i);
+            vm_barrier();
+            probs();
+            wait_chunk(i + 3u < n ? 1u : 0u);  // chunk i + 2
+            vm_barrier();
+        }
+        pv(n - 1u);
+    }
+
+    // ---- the split's partial: o / l in fp16 with (m, l); an empty split stores 0 ----
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
+    vm_barrier();
+    if (lane < 16) pm_s[64 * pb + 16 * hm + lane] = l_run;
+    vm_barrier();
+    const size_t bh = (size_t)b * a.nh + hbase;
+    if (pb == 0 && lane < 16) {
+        float* ml = a.part_ml + ((bh + 16u * hm + lane) * a.splits + sp) * 2u;
+        ml[0] = m_run;
+        ml[1] = pm_s[16 * hm + lane] + pm_s[64 + 16 * hm + lane];
+    }
+    // through LDS (the chunks are consumed: every wave is past its last P.V), so that a head's LR values go
+    // out as whole lines: 8-byte stores from the accumulators' layout, 32 bytes at a time, took 5.5 us
+    constexpr uint32_t kOPitch = LR + 8u;
+    static_assert(64u * kOPitch * 2u <= 4u * kBuf, "O fits the chunk buffers");
+    uint16_t* o_s = (uint16_t*)vm_smem;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        const int hh = 16 * h + col;
+        const float lh = pm_s[hh] + pm_s[64 + hh];
+        const float inv = lh > 0.0f ? 1.0f / lh : 0.0f;
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            uint16_t o[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = __builtin_bit_cast(uint16_t, (_Float16)(o_acc[h][nt][i] * inv));
+            *(uint2*)(o_s + (uint32_t)hh * kOPitch + 64 * wave + 16 * nt + 4 * grp) =
+                make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
+        }
+    }
+    vm_barrier();
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {  // a wave's 8 heads: 64 lanes x 16 bytes each
+        const uint32_t hh = 8u * (uint32_t)wave + (uint32_t)r;
+        *(uint4*)(a.part_o + ((bh + hh) * a.splits + sp) * LR + 8 * lane) = *(const uint4*)(o_s + hh * kOPitch + 8 * lane);
+    }
+}
+
 // LSE merge of the split partials of one (head, sequence) -> ctx[b][h][LR] fp32. A workgroup covers
 // 128 latent dimensions of its (head, sequence) (grid z), one per thread. The first NL splits'
 // loads are issued before the split weights are computed (they do not depend on them), then NL at
@@ -1134,14 +1444,32 @@ hipError_t vx_mla_attn_launch_t(const VxMlaAttnArgs& a, uint32_t batch, hipStrea
     return hipGetLastError();
 }
 
+hipError_t vx_mla_attn64_launch(const VxMlaAttnArgs& a, uint32_t batch, hipStream_t st) {
+    constexpr size_t lds = vx_mla_attn64_lds<512, 64>();
+    static bool attr_set = false;
+    if (!attr_set) {
+        if (hipFuncSetAttribute((const void*)vx_mla_attn64_kernel<512, 64>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds) != hipSuccess) {
+            (void)hipGetLastError();
+            return hipErrorInvalidValue;
+        }
+        attr_set = true;
+    }
+    const uint32_t items = a.splits * batch * (a.nh / 64u);
+    hipLaunchKernelGGL((vx_mla_attn64_kernel<512, 64>), dim3((items + 7u) / 8u * 8u), dim3(512), lds, st, a, batch);
+    return hipGetLastError();
+}
+
 hipError_t vx_launch_mla_attn(const VxMlaAttnArgs& a, uint32_t lr, uint32_t dr, uint32_t batch, hipStream_t st) {
     if (a.splits == 0 || a.splits > 64 || (a.s_cap & 31u) || a.s_cap < a.s_max || a.nh % 16u || dr != 64u)
         return hipErrorInvalidValue;
     // 4-wave workgroups (32 heads) where 8-wave ones (64 heads) would leave CUs idle: B=1 at 64
     // splits, 12.7 against 16.8 us (2-wave ones: 16.5)
-    if (lr == 512 && a.nh % 64u == 0 && (uint64_t)a.splits * batch * (a.nh / 64u) < 256u)
+    // (or a split's rows pass the 32-bit offsets of the 64-head kernel's loads)
+    if (lr == 512 && a.nh % 64u == 0 &&
+        ((uint64_t)a.splits * batch * (a.nh / 64u) < 256u || (uint64_t)a.s_cap * 1152u / a.splits + 65536u >= 1ull << 32))
         return vx_mla_attn_launch_t<512, 64, 2, 2>(a, batch, st);
-    if (lr == 512 && a.nh % 64u == 0) return vx_mla_attn_launch_t<512, 64, 4, 2>(a, batch, st);
+    if (lr == 512 && a.nh % 64u == 0) return vx_mla_attn64_launch(a, batch, st);
     if (lr == 128 && a.nh % 16u == 0) return vx_mla_attn_launch_t<128, 64, 1, 2>(a, batch, st);
     return hipErrorInvalidValue;
 }

@@ -75,6 +75,14 @@ __device__ __forceinline__ vm_h8 vm_f32x8_to_h8(float4 lo, float4 hi) {
     return r;
 }
 
+// A weight word read once per step: past the caches (NT), or through them.
+template <bool NT>
+__device__ __forceinline__ uint4 vm_ldw(const uint4* p) {
+    if constexpr (!NT) return *p;
+    const vm_u4 v = __builtin_nontemporal_load((const vm_u4*)p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 __device__ __forceinline__ float vm_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // The seeded N(0, sigma) value of the oracle's vxo_normal: an exact integer times coef.
@@ -276,7 +284,7 @@ __device__ __forceinline__ void vm_merge_stage(const VxF8GemmArgs& a, uint32_t g
     if (tid < lr) ((uint16_t*)smem)[tid] = __builtin_bit_cast(uint16_t, (_Float16)acc);
 }
 
-template <int KW, bool XF32>
+template <int KW, bool XF32, bool NT>
 __device__ __forceinline__ void vm_f8gemv_body(const VxF8GemmArgs& a) {
     extern __shared__ __align__(16) unsigned char vm_smem[];
     if ((a.active_mask & 1ULL) == 0ULL) return;
@@ -294,7 +302,7 @@ __device__ __forceinline__ void vm_f8gemv_body(const VxF8GemmArgs& a) {
     const uint32_t wl = w1 > w0 ? w1 - 1u : w0;
     uint4 wr[D];
 #pragma unroll
-    for (int u = 0; u < D; ++u) wr[u] = W[(size_t)min(w0 + (uint32_t)u, wl) * 64u];
+    for (int u = 0; u < D; ++u) wr[u] = vm_ldw<NT>(W + (size_t)min(w0 + (uint32_t)u, wl) * 64u);
     // x over the split's k-range -> LDS as fp16 (8 elements per thread and pass); with a gain, x is
     // first RMSNorm'd over its whole row (every workgroup sums the row's squares itself), in the
     // operation order of the batched RMSNorm kernel: (x * inv_rms) * gain, rounded to fp16
@@ -401,7 +409,7 @@ __device__ __forceinline__ void vm_f8gemv_body(const VxF8GemmArgs& a) {
                 }
                 acc = fmaf(S[kt >> 1], d, acc);
             }
-            wr[u] = W[(size_t)min(kt + (uint32_t)D, wl) * 64u];
+            wr[u] = vm_ldw<NT>(W + (size_t)min(kt + (uint32_t)D, wl) * 64u);
         }
     }
     // the row's four k-groups, then the KW waves of the tile
@@ -427,9 +435,9 @@ __device__ __forceinline__ void vm_f8gemv_body(const VxF8GemmArgs& a) {
     }
 }
 
-template <int KW, bool XF32>
+template <int KW, bool XF32, bool NT>
 __global__ __launch_bounds__(64 * kFGWaves) void vx_f8gemv_kernel(VxF8GemmArgs a) {
-    vm_f8gemv_body<KW, XF32>(a);
+    vm_f8gemv_body<KW, XF32, NT>(a);
 }
 
 // The same structure for 2..16 sequences on the matrix cores: the workgroup stages its split's
@@ -437,7 +445,7 @@ __global__ __launch_bounds__(64 * kFGWaves) void vx_f8gemv_kernel(VxF8GemmArgs a
 // the A operands of its two MFMAs (row col, k-elements 16 grp + 0..7 and + 8..15) from LDS and the B
 // operands from its weight word, then acc += block scale * the tile's product. KW waves per row tile
 // meet in LDS; the first writes 16 rows x the batch's sequences.
-template <int KW, bool XF32>
+template <int KW, bool XF32, bool NT>
 __global__ __launch_bounds__(64 * kFGWaves) void vx_f8gemm_x_kernel(VxF8GemmArgs a) {
     extern __shared__ __align__(16) unsigned char vm_smem[];
     if ((a.active_mask & 1ULL) == 0ULL) return;
@@ -453,7 +461,7 @@ __global__ __launch_bounds__(64 * kFGWaves) void vx_f8gemm_x_kernel(VxF8GemmArgs
     const uint32_t wl = w1 > w0 ? w1 - 1u : w0;
     uint4 wr[D];
 #pragma unroll
-    for (int u = 0; u < D; ++u) wr[u] = W[(size_t)min(w0 + (uint32_t)u, wl) * 64u];
+    for (int u = 0; u < D; ++u) wr[u] = vm_ldw<NT>(W + (size_t)min(w0 + (uint32_t)u, wl) * 64u);
     // x rows 0..15 over the split's k-range -> LDS fp16, rows XR elements apart (16 bytes of padding
     // per row: the 16 rows' operand reads fall in different banks)
     uint4* xs = (uint4*)vm_smem;
@@ -506,7 +514,7 @@ __global__ __launch_bounds__(64 * kFGWaves) void vx_f8gemm_x_kernel(VxF8GemmArgs
             acc += sprev * tprev;
             tprev = t;
             sprev = kt < w1 ? sr[u] : 0.0f;
-            wr[u] = W[(size_t)min(kt + (uint32_t)D, wl) * 64u];
+            wr[u] = vm_ldw<NT>(W + (size_t)min(kt + (uint32_t)D, wl) * 64u);
             sr[u] = Sv[min(kt + (uint32_t)D, wl) >> 1];
         }
     }
@@ -538,16 +546,30 @@ template <int KW>
 void vx_f8gemm_x_launch_t(const VxF8GemmArgs& a, uint32_t groups, size_t lds, hipStream_t st) {
     constexpr int TPW = kFGWaves / KW;
     const dim3 grid((a.n_rt + TPW - 1) / TPW, a.ksplit, groups), block(64 * kFGWaves);
-    if (a.x_f32) hipLaunchKernelGGL((vx_f8gemm_x_kernel<KW, true>), grid, block, lds, st, a);
-    else hipLaunchKernelGGL((vx_f8gemm_x_kernel<KW, false>), grid, block, lds, st, a);
+    // Ungrouped matrices (7-117 MB) pass the caches, which keep the activations: at DeepSeek-V3 W_o 25.6 ->
+    // 22.4 us for 16 sequences, 22.5 -> 21.0 for one (kernel trace). The per-head groups' 64 KB do not:
+    // W_uk^T would go 3.5 -> 4.3, W_uv 5.2 -> 5.9 us.
+    if (groups > 1u) {
+        if (a.x_f32) hipLaunchKernelGGL((vx_f8gemm_x_kernel<KW, true, false>), grid, block, lds, st, a);
+        else hipLaunchKernelGGL((vx_f8gemm_x_kernel<KW, false, false>), grid, block, lds, st, a);
+    } else {
+        if (a.x_f32) hipLaunchKernelGGL((vx_f8gemm_x_kernel<KW, true, true>), grid, block, lds, st, a);
+        else hipLaunchKernelGGL((vx_f8gemm_x_kernel<KW, false, true>), grid, block, lds, st, a);
+    }
 }
 
 template <int KW>
 void vx_f8gemv_launch_t(const VxF8GemmArgs& a, uint32_t groups, size_t lds, hipStream_t st) {
     constexpr int TPW = kFGWaves / KW;
     const dim3 grid((a.n_rt + TPW - 1) / TPW, a.ksplit, groups), block(64 * kFGWaves);
-    if (a.x_f32) hipLaunchKernelGGL((vx_f8gemv_kernel<KW, true>), grid, block, lds, st, a);
-    else hipLaunchKernelGGL((vx_f8gemv_kernel<KW, false>), grid, block, lds, st, a);
+    // (the weights' cache policy as above)
+    if (groups > 1u) {
+        if (a.x_f32) hipLaunchKernelGGL((vx_f8gemv_kernel<KW, true, false>), grid, block, lds, st, a);
+        else hipLaunchKernelGGL((vx_f8gemv_kernel<KW, false, false>), grid, block, lds, st, a);
+    } else {
+        if (a.x_f32) hipLaunchKernelGGL((vx_f8gemv_kernel<KW, true, true>), grid, block, lds, st, a);
+        else hipLaunchKernelGGL((vx_f8gemv_kernel<KW, false, true>), grid, block, lds, st, a);
+    }
 }
 
 template <int MT, int MR>
@@ -768,7 +790,7 @@ __global__ __launch_bounds__(64 * kFGWaves) void vx_f8gemv_prep_kernel(VxF8GemmA
         vm_prep_latent<64 * kFGWaves>(p, 0u, (float*)vm_smem);
         return;
     }
-    vm_f8gemv_body<KW, true>(g);
+    vm_f8gemv_body<KW, true, true>(g);
 }
 
 __global__ __launch_bounds__(1024) void vx_mla_prep_kernel(VxMlaPrepArgs a) {

@@ -299,3 +299,12 @@ def test_prefill_llama3_8b_full_depth_128_rows_vs_oracle(oracle):
         assert d < LOGIT_TOL, (pos, d)
     print(f"[llama3_8b prefill 128 rows, 32 layers] worst logits maxabs {worst:.3e}", flush=True)
     ref.close()
+
+
+@pytest.mark.parametrize("chunk,rows", [(128, 129), (65, 193), (128, 300)])
+def test_prefill_row_blocks_and_long_contexts_vs_oracle(oracle, chunk, rows):
+    """Chunks just past 64 rows (their GEMMs split K for two row blocks) and rows attending past 128 positions
+    (8-wave attention workgroups), down to a 1-row tail: a narrow layer with 7 q heads per KV head."""
+    cfg = dict(vocab_size=512, hidden_dim=384, intermediate_dim=640, num_heads=14, num_kv_heads=2, head_dim=128,
+               rms_norm_eps=1e-6, rope_theta=1000000.0, qkv_bias=1, tied_lm_head=1)
+    _prefill_vs_oracle(oracle, cfg, 2, chunk, rows, [(0, rows)], rows + 20, seed=83, decode_steps=1)

@@ -63,12 +63,12 @@ uint32_t vx_mgemm_ksplit(const VxMatPlan& m) {
     return ks ? ks : 1u;
 }
 
-// K splits of the QKV GEMM over more than 16 rows (the LDS-shared GEMM, 8 tiles per workgroup): as
-// many as keep the grid within one round of 256 workgroups, where a partial second round would add
-// a whole workgroup's time (Llama-3-8B QKV at 128 rows: 48 x 6 workgroups 26.6 us, 48 x 5 21.9 us;
-// Qwen2.5-7B at 32 sequences: 36 x 8 9.7 us, 36 x 7 8.3 us).
-uint32_t vx_pgemm_ksplit(const VxMatPlan& m) {
-    const uint32_t wgs = vx_pgemm_grid(m.m_tiles);
+// K splits of a GEMM over more than 16 rows (the LDS-shared GEMM, 8 tiles per workgroup, row_blocks
+// workgroups over the rows): as many as keep the grid within one round of 256 workgroups, where a partial
+// second round would add a whole workgroup's time (Llama-3-8B QKV at 128 rows: 48 x 6 workgroups 26.6 us,
+// 48 x 5 21.9 us; Qwen2.5-7B at 32 sequences: 36 x 8 9.7 us, 36 x 7 8.3 us).
+uint32_t vx_pgemm_ksplit(const VxMatPlan& m, uint32_t row_blocks) {
+    const uint32_t wgs = vx_pgemm_grid(m.m_tiles) * row_blocks;
     uint32_t ks = wgs ? 256u / wgs : 1u;
     if (ks > 8u) ks = 8u;
     if (ks > m.m_grp) ks = m.m_grp;
@@ -107,6 +107,11 @@ struct VeloxHipModel {
     uint64_t a_bpart_r = 0;
     uint32_t ksplit_o = 1, ksplit_down = 1, ksplit_qkv = 1;
     uint32_t ksplit_qkv_wide = 1;  // QKV over more than 16 rows
+    // over more than 64 rows, two 64-row blocks of workgroups: QKV, o_proj, down split less, so that one
+    // round holds both blocks and half the partials are written and folded (whole prefill step: Llama-3-8B at
+    // 128 rows QKV 5 -> 2 splits 642 -> 637 us, o_proj 8 -> 4 636, down 8 -> 4 638; Qwen2.5-7B at 1000 rows
+    // 7 -> 3, 8 -> 4, 8 -> 4: 2970 -> 2938, 2933, 2967)
+    uint32_t ksplit_qkv_128 = 1, ksplit_o_128 = 1, ksplit_down_128 = 1;
     // fp16 activation operands of the batched GEMMs (over the MFMA-layout copies): element k of row m
     // at m * x_ld + (k / 32) * x_bs + k % 32, block-major [k / 32][16-row-padded rows][32] (one operand
     // load = 1 KiB contiguous)
@@ -553,7 +558,10 @@ int velox_hip_model_create(const VeloxHipModelConfig* cfg, VeloxHipModel** out) 
         M->a_bpart_r = take(8 * B * (H > qd + 2 * kvd ? H : qd + 2 * kvd) * 4);
         M->a_prows = take(B * sizeof(VeloxDecodeState));
         M->ksplit_qkv = vx_mgemm_ksplit(M->layers[0].qkv);
-        M->ksplit_qkv_wide = vx_pgemm_ksplit(M->layers[0].qkv);
+        M->ksplit_qkv_wide = vx_pgemm_ksplit(M->layers[0].qkv, 1u);
+        M->ksplit_qkv_128 = vx_pgemm_ksplit(M->layers[0].qkv, 2u);
+        M->ksplit_o_128 = vx_pgemm_ksplit(M->layers[0].o, 2u);
+        M->ksplit_down_128 = vx_pgemm_ksplit(M->layers[0].down, 2u);
         M->ksplit_o = vx_mgemm_ksplit(M->layers[0].o);
         M->ksplit_down = vx_mgemm_ksplit(M->layers[0].down);
     }
@@ -1138,6 +1146,9 @@ void vx_rows_forward(const VeloxHipModel* M, VeloxHipArena* A, const VeloxDecode
     float* qkv = (float*)(act + M->a_bqkv);
     float* part_r = (float*)(act + M->a_bpart_r);
     const uint64_t pstride = (uint64_t)M->rows * H;
+    const uint32_t ks_qkv = n > 64u ? M->ksplit_qkv_128 : n > 16u ? M->ksplit_qkv_wide : M->ksplit_qkv;
+    const uint32_t ks_o = n > 64u ? M->ksplit_o_128 : M->ksplit_o;
+    const uint32_t ks_down = n > 64u ? M->ksplit_down_128 : M->ksplit_down;
     auto gemm = [&](const VxMatPlan& p, const VxBGemmArgs& ga, int epi) {
         return vx_launch_mgemm(vx_mview(A, p), ga, epi, st);
     };
@@ -1178,7 +1189,7 @@ void vx_rows_forward(const VeloxHipModel* M, VeloxHipArena* A, const VeloxDecode
     for (uint32_t l = 0; l < c.num_layers; ++l) {
         const VxLayerPlan& L = M->layers[l];
         // the previous layer's down projection left its K-split partials (none before layer 0)
-        vx_record(vx_launch_bnorm(h, H, l && M->ksplit_down > 1 ? part_r : nullptr, M->ksplit_down, pstride,
+        vx_record(vx_launch_bnorm(h, H, l && ks_down > 1 ? part_r : nullptr, ks_down, pstride,
                                   vecp(L.attn_norm), H, c.rms_norm_eps, xa, M->x_ld, M->x_bs, n, mask, st));
         std::memset(&g, 0, sizeof(g));
         g.batch = n;
@@ -1189,7 +1200,6 @@ void vx_rows_forward(const VeloxHipModel* M, VeloxHipArena* A, const VeloxDecode
         g.bias = c.qkv_bias ? vecp(L.bias) : nullptr;
         g.y = qkv;
         g.ldy = qd + 2 * kvd;
-        const uint32_t ks_qkv = n > 16u ? M->ksplit_qkv_wide : M->ksplit_qkv;
         if (ks_qkv > 1) {  // K-split partials, then their sum + bias
             g.ksplit = ks_qkv;
             g.part = part_r;
@@ -1217,11 +1227,11 @@ void vx_rows_forward(const VeloxHipModel* M, VeloxHipArena* A, const VeloxDecode
         g.xbs = M->x_bs;
         g.y = h;
         g.ldy = H;
-        g.ksplit = M->ksplit_o;
+        g.ksplit = ks_o;
         g.part = part_r;
         g.pstride = pstride;
         vx_record(gemm(L.o, g, VX_EPI_RESID));
-        vx_record(vx_launch_bnorm(h, H, M->ksplit_o > 1 ? part_r : nullptr, M->ksplit_o, pstride, vecp(L.mlp_norm), H,
+        vx_record(vx_launch_bnorm(h, H, ks_o > 1 ? part_r : nullptr, ks_o, pstride, vecp(L.mlp_norm), H,
                                   c.rms_norm_eps, xa, M->x_ld, M->x_bs, n, mask, st));
         std::memset(&g, 0, sizeof(g));
         g.batch = n;
@@ -1241,12 +1251,12 @@ void vx_rows_forward(const VeloxHipModel* M, VeloxHipArena* A, const VeloxDecode
         g.xbs = M->x_bs;
         g.y = h;
         g.ldy = H;
-        g.ksplit = M->ksplit_down;
+        g.ksplit = ks_down;
         g.part = part_r;
         g.pstride = pstride;
         vx_record(gemm(L.down, g, VX_EPI_RESID));
     }
-    vx_record(vx_launch_bnorm(h, H, M->ksplit_down > 1 ? part_r : nullptr, M->ksplit_down, pstride,
+    vx_record(vx_launch_bnorm(h, H, ks_down > 1 ? part_r : nullptr, ks_down, pstride,
                               vecp(M->final_norm), H, c.rms_norm_eps, xa, M->x_ld, M->x_bs, n, mask, st));
     std::memset(&g, 0, sizeof(g));
     g.batch = n;

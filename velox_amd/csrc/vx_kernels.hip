@@ -743,10 +743,14 @@ hipError_t vx_attn_launch_w(const VxAttnArgs& a, hipStream_t st) {
 template <int D, int G, bool PS>
 hipError_t vx_attn_launch_ps(const VxAttnArgs& a, hipStream_t st) {
     if constexpr (PS) {
-        // prefill chunks: 16 / G rows per workgroup (4-wave workgroups)
+        // prefill chunks: 16 / G rows per workgroup; 4 waves while they take every 32-position chunk in one
+        // pass, 8 beyond (a 128-row chunk is about one workgroup per CU: at 129-1000 positions of Qwen2.5-7B
+        // 18.3 -> 15.7 us median, 23.3 -> 20.0 in the last chunk)
         constexpr int R = 16 / G;
         if constexpr (R > 1)
-            if (a.prefill) return vx_attn_launch_w<D, G, PS, 4, R>(a, st);
+            if (a.prefill)
+                return a.max_len > 4u * 32u ? vx_attn_launch_w<D, G, PS, 8, R>(a, st)
+                                            : vx_attn_launch_w<D, G, PS, 4, R>(a, st);
         // 4 waves, two workgroups per CU, where 8-wave workgroups (one per CU) would need a second
         // round and 4 waves still take every 32-position chunk a split can attend in one pass (the
         // prefill chunks of short prompts: 64 rows x 8 KV heads = 512 workgroups, <= 128 positions)

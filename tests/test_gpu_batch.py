@@ -132,6 +132,12 @@ def test_batch_decode_qwen_bias_32_vs_oracle(oracle):
     _batch_vs_oracle(oracle, QWEN_SMALL_VOCAB, QWEN_SMALL_VOCAB, 1, 32, 2, 8, seed=52, starts=[0] * 32)
 
 
+@pytest.mark.parametrize("batch", [2, 16])
+def test_batch_decode_splits_of_16_rows_vs_oracle(oracle, batch):
+    """The K splits of up to 16 rows (o_proj 112 grid rows x 4, down x 4, QKV 144 x 3) at both ends of their range."""
+    _batch_vs_oracle(oracle, QWEN_SMALL_VOCAB, QWEN_SMALL_VOCAB, 1, batch, 2, 8, seed=53, starts=[0] * batch)
+
+
 def test_batch_run_graph_matches_eager(oracle):
     """velox_hip_run with batch > 1 (hipGraph of the batched step) produces sequence 0's tokens of an
     eager batched decode of the same seeded prompts."""

@@ -52,12 +52,23 @@ struct VxLayerPlan {
     uint64_t attn_norm = 0, mlp_norm = 0, bias = 0;
 };
 
-// K splits of a batched GEMM over the MFMA layout: enough grid rows for about 1024 workgroups (two
+// K splits of o_proj and down over 17-64 rows: enough grid rows for about 1024 workgroups (two
 // 16-row tiles each, its 4 waves splitting K again), at most 8 (the partials a batched RMSNorm or
 // the partial sum folds in) and at most one group of 4 blocks per split.
 uint32_t vx_mgemm_ksplit(const VxMatPlan& m) {
     const uint32_t wgs = vx_mgemm_grid(m.m_tiles);
     uint32_t ks = (1024u + wgs - 1u) / wgs;
+    if (ks > 8u) ks = 8u;
+    if (ks > m.m_grp) ks = m.m_grp;
+    return ks ? ks : 1u;
+}
+
+// K splits over up to 16 rows (the 4-wave GEMM): whole splits within 512 workgroups, two per CU. Against the
+// ~1024 of the rule above, half the partials to write and fold and longer streams per wave: two-layer stacks at
+// 8 sequences 162.4 -> 160.2 us (Qwen2.5-7B), 163.9 -> 162.1 (Llama-3-8B), 327.7 -> 323.0 (Qwen2-72B), SmolLM as
+// before; at 32 sequences of Qwen2.5-7B (the LDS-shared GEMM) fewer splits lose (o_proj 8 -> 4: 446 -> 449 us).
+uint32_t vx_mgemm_ksplit16(const VxMatPlan& m) {
+    uint32_t ks = 512u / vx_mgemm_grid(m.m_tiles);
     if (ks > 8u) ks = 8u;
     if (ks > m.m_grp) ks = m.m_grp;
     return ks ? ks : 1u;
@@ -107,6 +118,7 @@ struct VeloxHipModel {
     uint64_t a_bpart_r = 0;
     uint32_t ksplit_o = 1, ksplit_down = 1, ksplit_qkv = 1;
     uint32_t ksplit_qkv_wide = 1;  // QKV over more than 16 rows
+    uint32_t ksplit_o16 = 1, ksplit_down16 = 1;  // o_proj and down of up to 16 rows
     // over more than 64 rows, two 64-row blocks of workgroups: QKV, o_proj, down split less, so that one
     // round holds both blocks and half the partials are written and folded (whole prefill step: Llama-3-8B at
     // 128 rows QKV 5 -> 2 splits 642 -> 637 us, o_proj 8 -> 4 636, down 8 -> 4 638; Qwen2.5-7B at 1000 rows
@@ -557,7 +569,9 @@ int velox_hip_model_create(const VeloxHipModelConfig* cfg, VeloxHipModel** out) 
         // K-split partials: [8][rows][max(hidden, q/k/v width)]
         M->a_bpart_r = take(8 * B * (H > qd + 2 * kvd ? H : qd + 2 * kvd) * 4);
         M->a_prows = take(B * sizeof(VeloxDecodeState));
-        M->ksplit_qkv = vx_mgemm_ksplit(M->layers[0].qkv);
+        M->ksplit_qkv = vx_mgemm_ksplit16(M->layers[0].qkv);
+        M->ksplit_o16 = vx_mgemm_ksplit16(M->layers[0].o);
+        M->ksplit_down16 = vx_mgemm_ksplit16(M->layers[0].down);
         M->ksplit_qkv_wide = vx_pgemm_ksplit(M->layers[0].qkv, 1u);
         M->ksplit_qkv_128 = vx_pgemm_ksplit(M->layers[0].qkv, 2u);
         M->ksplit_o_128 = vx_pgemm_ksplit(M->layers[0].o, 2u);
@@ -1147,8 +1161,8 @@ void vx_rows_forward(const VeloxHipModel* M, VeloxHipArena* A, const VeloxDecode
     float* part_r = (float*)(act + M->a_bpart_r);
     const uint64_t pstride = (uint64_t)M->rows * H;
     const uint32_t ks_qkv = n > 64u ? M->ksplit_qkv_128 : n > 16u ? M->ksplit_qkv_wide : M->ksplit_qkv;
-    const uint32_t ks_o = n > 64u ? M->ksplit_o_128 : M->ksplit_o;
-    const uint32_t ks_down = n > 64u ? M->ksplit_down_128 : M->ksplit_down;
+    const uint32_t ks_o = n > 64u ? M->ksplit_o_128 : n > 16u ? M->ksplit_o : M->ksplit_o16;
+    const uint32_t ks_down = n > 64u ? M->ksplit_down_128 : n > 16u ? M->ksplit_down : M->ksplit_down16;
     auto gemm = [&](const VxMatPlan& p, const VxBGemmArgs& ga, int epi) {
         return vx_launch_mgemm(vx_mview(A, p), ga, epi, st);
     };

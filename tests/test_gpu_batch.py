@@ -312,6 +312,14 @@ def test_gemm_m_swiglu(hiplib, oracle, dev, F, H, batch, bm):
     assert rms(got - want) < 5e-4 * rms(want)
 
 
+@pytest.mark.parametrize("F,H,batch", [(16385, 608, 17), (20480, 608, 48), (20480, 416, 64), (20481, 608, 33), (8192, 416, 32),
+                                       (8193, 608, 32), (4090, 608, 50), (8192, 384, 20)])
+def test_gemm_m_workgroup_shapes(hiplib, oracle, dev, F, H, batch):
+    """Gate/up at the edges of the workgroup shapes: 10-tile workgroups from 2050 tiles to 2560, the two-tile ones
+    with K in four parts up to 512 workgroups and from 4 groups of K (parts of two groups and empty ones)."""
+    test_gemm_m_swiglu(hiplib, oracle, dev, F, H, batch, 1)
+
+
 def test_gemm_m_rejects_bad_arguments(hiplib, oracle, dev):
     blocks = _weights(oracle, 64, 576, 9)
     t = TiledQ4(hiplib, dev, blocks, 64, 576)

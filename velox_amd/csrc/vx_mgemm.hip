@@ -326,23 +326,23 @@ __global__ __launch_bounds__(kMThreads) void vx_mgemm_kernel(VxMMat w, VxBGemmAr
     }
 }
 
-// ---- the GEMM for 17-64 activation rows (prefill chunks, 17-32 sequences) ----
-// A workgroup owns 8 tiles over all MT row tiles and its grid row's K range, which its two halves
-// of 4 waves split (the first half takes the first ceil(n / 2) groups); in each half wave w owns
-// tiles 2w, 2w + 1 (a gate/up pair for SWIGLU). Per group of 4 blocks a half stages the group's
-// 4 x MT activation tiles (1 KiB each) once in LDS, in the lane order of the MFMA A operand, and
-// its 4 waves read them from there for both their tiles: a quarter of the activation loads of the
+// ---- the GEMM for 17-128 activation rows (prefill chunks, 17-32 sequences) ----
+// A workgroup owns 2 PW tiles over MT row tiles and its grid row's K range, which its KH parts of PW
+// waves split in turn (parts of ceil(n / KH) groups, the last ones shorter or empty); in each part
+// wave w owns tiles 2w, 2w + 1 (a gate/up pair for SWIGLU). Per group of 4 blocks a part stages the
+// group's 4 x MT activation tiles (1 KiB each) once in LDS, in the lane order of the MFMA A operand,
+// and its PW waves read them from there for both their tiles: 1 / PW of the activation loads of the
 // kernel above, whose waves split K and each load their own. Stages are double-buffered, one
-// barrier per group; the weights are loaded 4 groups ahead and the activations 2 ahead. The two
-// halves put two waves on every SIMD, so one wave's VALU work partly overlaps the other's MFMAs
-// (with one 4-wave half, Llama's gate/up at 64 rows kept the matrix cores busy a third of its
+// barrier per group; the weights are loaded 4 groups ahead and the activations 2 ahead. Two
+// parts put two waves on every SIMD, so one wave's VALU work partly overlaps the other's MFMAs
+// (with one part of 4 waves, Llama's gate/up at 64 rows kept the matrix cores busy a third of its
 // 42 us); their sums meet in LDS at the end. The arithmetic is the kernel above's: exact block
 // products, the block scale applied in fp32 (4 VALU per MFMA). Splitting each weight d (q - 8)
 // exactly into two fp16 MFMA operands instead (hi = fp16(d (q - 8)), lo = the fused residual) needs
 // no scale multiply-adds but twice the MFMAs, and measured slower: on gfx950 a wave's MFMAs and
 // another wave's VALU instructions on the same SIMD take about the MFMA time plus half the VALU
 // time (timed with MFMA-only and VALU-only waves sharing the SIMDs).
-constexpr int kPNT = 2, kPTiles = kPNT * kMWaves;  // tiles per wave, per workgroup
+constexpr int kPNT = 2, kPTiles = kPNT * kMWaves;  // tiles per wave, per workgroup of 4 waves a part
 constexpr int kPRing = 4;                           // weight register sets: groups loaded ahead
 
 template <int P>
@@ -350,27 +350,25 @@ struct vx_ic {
     static constexpr int value = P;
 };
 
-template <int EPI, int MT, int KH>
-__global__ __launch_bounds__(kMThreads * KH) void vx_pgemm_kernel(VxMMat w, VxBGemmArgs a) {
+template <int EPI, int MT, int KH, int PW>
+__global__ __launch_bounds__(64 * PW * KH) void vx_pgemm_kernel(VxMMat w, VxBGemmArgs a) {
     if ((a.active_mask & 1ULL) == 0ULL) return;
-    constexpr int NT = kPNT, SU = 4 * MT, UPW = SU / kMWaves;  // 1 KiB units per group, per wave
-    static_assert(SU % kMWaves == 0, "whole units per wave");
-    static_assert(KH == 1 || KH == 2, "one or two K halves");
-    static_assert(sizeof(vx_mh8) * 2 * 2 * SU * 64 >= sizeof(vx_mf4) * kMWaves * NT * MT * 64, "reduction fits");
+    constexpr int NT = kPNT, SU = 4 * MT, UPW = (SU + PW - 1) / PW;  // 1 KiB units per group, per wave
+    static_assert(sizeof(vx_mh8) * KH * 2 * SU * 64 >= (KH - 1) * sizeof(vx_mf4) * PW * NT * MT * 64, "reduction fits");
     extern __shared__ __align__(16) unsigned char vx_psmem[];
-    vx_mh8(*xs)[2][SU][64] = (vx_mh8(*)[2][SU][64])vx_psmem;  // [half][stage][block * MT + row tile][lane]
+    vx_mh8(*xs)[2][SU][64] = (vx_mh8(*)[2][SU][64])vx_psmem;  // [part][stage][block * MT + row tile][lane]
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kh = KH == 1 ? 0 : wv / kMWaves, wave = wv % kMWaves;  // K half, wave within the half
+    const int kh = KH == 1 ? 0 : wv / PW, wave = wv % PW;  // K part, wave within the part
     const int row = lane & 15, g = lane >> 4;
-    const uint32_t T0 = blockIdx.x * (uint32_t)kPTiles + 2u * (uint32_t)wave;  // this wave's first tile
+    const uint32_t T0 = blockIdx.x * (uint32_t)(kPNT * PW) + 2u * (uint32_t)wave;  // this wave's first tile
     const uint32_t r0 = blockIdx.z * (uint32_t)(16 * MT);  // the workgroup's first activation row
     const uint32_t ng = w.n_grp;
     const uint32_t jg0 = blockIdx.y * ng / gridDim.y, j1 = (blockIdx.y + 1u) * ng / gridDim.y;
     const uint32_t jl = j1 - 1u;  // j1 > jg0: the launcher keeps ksplit <= n_grp
-    // both halves run ns steps (the barriers are the workgroup's); the second half's last step has
-    // no group when the count is odd
+    // every part runs ns steps (the barriers are the workgroup's); the last parts' last steps have no
+    // group where KH does not divide the count
     const uint32_t ns = (j1 - jg0 + (uint32_t)KH - 1u) / (uint32_t)KH;
-    const uint32_t j0 = jg0 + (uint32_t)kh * ns, nj = kh ? (j1 - jg0) - ns : ns;
+    const uint32_t j0 = jg0 + (uint32_t)kh * ns, nj = j0 < j1 ? min(j1 - j0, ns) : 0u;
 
     // tiles past the matrix re-read its last tile, rows past the batch the last row, blocks past k
     // (zero codes and scales) the last real block: every load is in bounds and unconditional
@@ -382,13 +380,14 @@ __global__ __launch_bounds__(kMThreads * KH) void vx_pgemm_kernel(VxMMat w, VxBG
         cp[nt] = (const vx_mu4*)w.codes + (size_t)t * ng * 64u + lane;
         sp[nt] = (const vx_mu2*)w.scales + (size_t)t * ng * 16u + row;
     }
-    // the wave stages units wave, wave + 4, ...: unit u is block u / MT, row tile u % MT; lane
+    // the wave stages units wave, wave + PW, ... (past the last unit that one again, the same bytes from
+    // each wave, so that all waves have the same loads in flight): unit u is block u / MT, row tile u % MT; lane
     // (row, g) moves elements 8 g .. 8 g + 7 of the tile's row, the A operand it later reads
     const uint16_t* xsrc[UPW];
     uint32_t xblk[UPW];
 #pragma unroll
     for (int i = 0; i < UPW; ++i) {
-        const int u = wave + kMWaves * i;
+        const int u = min(wave + PW * i, SU - 1);
         xblk[i] = (uint32_t)(u / MT);
         xsrc[i] = a.x16 + (size_t)min(r0 + (uint32_t)(16 * (u % MT) + row), a.batch - 1u) * a.ldx + 8 * g;
     }
@@ -428,7 +427,7 @@ __global__ __launch_bounds__(kMThreads * KH) void vx_pgemm_kernel(VxMMat w, VxBG
     auto store_x = [&](auto pc, int s) {
         constexpr int p = decltype(pc)::value;
 #pragma unroll
-        for (int i = 0; i < UPW; ++i) xs[kh][s][wave + kMWaves * i][lane] = xr[p][i];
+        for (int i = 0; i < UPW; ++i) xs[kh][s][min(wave + PW * i, SU - 1)][lane] = xr[p][i];
     };
     // block b of the group: c = mfma(x, q - 8, 0), acc += d_b c -- the arithmetic of the kernel above.
     // Software-pipelined over (block, row tile): the MFMAs of one (b, mt) are issued before the
@@ -521,22 +520,24 @@ __global__ __launch_bounds__(kMThreads * KH) void vx_pgemm_kernel(VxMMat w, VxBG
     if (i + 1u < ns) step(vx_ic<1>{}, i + 1u);
     if (i + 2u < ns) step(vx_ic<2>{}, i + 2u);
 
-    // the second half's sums into LDS (the stages are free after the last step's barrier), added
-    // to the first half's in that order
-    if constexpr (KH == 2) {
-        vx_mf4(*red)[NT * MT][64] = (vx_mf4(*)[NT * MT][64])&xs[0][0][0][0];
+    // the other parts' sums into LDS (the stages are free after the last step's barrier), added
+    // to the first part's in their order
+    if constexpr (KH > 1) {
+        vx_mf4(*red)[PW][NT * MT][64] = (vx_mf4(*)[PW][NT * MT][64])&xs[0][0][0][0];
         if (kh) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) red[wave][nt * MT + mt][lane] = acc[nt][mt];
+                for (int mt = 0; mt < MT; ++mt) red[kh - 1][wave][nt * MT + mt][lane] = acc[nt][mt];
         }
         __syncthreads();
         if (kh) return;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
+        for (int h = 0; h < KH - 1; ++h)
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[nt][mt] += red[wave][nt * MT + mt][lane];
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) acc[nt][mt] += red[h][wave][nt * MT + mt][lane];
     }
 
     // ---- epilogues (every wave, its two tiles): lane holds acc[nt][mt][i] for activation row
@@ -612,34 +613,55 @@ namespace {
 
 constexpr int kMNT = 2;  // tiles per wave (a gate/up pair for SWIGLU)
 
-// Used for 17-128 rows (Qwen2.5-7B decode at 32 sequences: 9797-9850 -> 9972-10164 tok/s).
-// Two K halves per workgroup where the grid is at most one round of workgroups and each has 8 or
-// more groups (Llama-3-8B at 64 rows: gate/up 47.5 -> 36.2 us, down); one where the grid already
-// fills the CUs or the groups are few (QKV and o_proj split 5-8 ways over K, the LM head).
-template <int EPI, int MT, int KH>
-hipError_t vx_pgemm_launch_kh(const VxMMat& w, const VxBGemmArgs& a, dim3 grid, hipStream_t st) {
-    constexpr size_t lds = (size_t)KH * 2 * 4 * MT * 1024;  // [half][stage][4 MT activation tiles of 1 KiB]
+template <int EPI, int MT, int KH, int PW>
+hipError_t vx_pgemm_launch_kh(const VxMMat& w, const VxBGemmArgs& a, hipStream_t st) {
+    constexpr size_t lds = (size_t)KH * 2 * 4 * MT * 1024;  // [part][stage][4 MT activation tiles of 1 KiB]
     static bool attr_set = false;
     if (!attr_set) {
-        if (hipFuncSetAttribute((const void*)vx_pgemm_kernel<EPI, MT, KH>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute((const void*)vx_pgemm_kernel<EPI, MT, KH, PW>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds) != hipSuccess) {
             (void)hipGetLastError();
             return hipErrorInvalidValue;
         }
         attr_set = true;
     }
-    grid.z = (a.batch + 16u * MT - 1u) / (16u * MT);  // blocks of 16 MT activation rows
-    hipLaunchKernelGGL((vx_pgemm_kernel<EPI, MT, KH>), grid, dim3(KH * kMThreads), lds, st, w, a);
+    const dim3 grid((w.n_tiles + kPNT * PW - 1u) / (kPNT * PW), a.ksplit > 1u ? a.ksplit : 1u,
+                    (a.batch + 16u * MT - 1u) / (16u * MT));  // z: blocks of 16 MT activation rows
+    hipLaunchKernelGGL((vx_pgemm_kernel<EPI, MT, KH, PW>), grid, dim3(64 * KH * PW), lds, st, w, a);
     return hipGetLastError();
 }
 
+// Used for 17-128 rows (Qwen2.5-7B decode at 32 sequences: 9797-9850 -> 9972-10164 tok/s). What a
+// launch takes is its busiest CU's work (a CU holds one workgroup of two parts, or two of one part),
+// so the workgroup's shape follows the grid:
+//   - gate/up and the LM head where one wave's two tiles and 32 rows per workgroup still come to at
+//     most 512 workgroups: that, K split four ways. With 8 tiles a small matrix left most CUs idle:
+//     2048 rows of 3584 (16 workgroups) 20.4 -> 14.0 us at 32 rows; a Qwen2.5-7B layer with it 126.4 ->
+//     113.6 us at 32 rows and 205.5 -> 189 at 128; with 16000 rows (500 workgroups) 128.9 -> 122.5,
+//     but 169.5 -> 165 and 209 -> 235 at 64 and 128 rows (1000 and 2000 workgroups: activations read
+//     by too many); 8 layers of SmolLM at 17 rows 309 -> 306, 4 at 64 rows 217 -> 198.
+//   - gate/up whose 8-tile workgroups are more than one round, at up to 64 rows, while 10-tile ones
+//     are not (2049-2560 tiles): 5 waves a part, two parts. Qwen2.5-7B's 2368 tiles left 40 of 256
+//     CUs with two workgroups and the others waiting for them: 33.7 -> 27.1 us at 32 rows; two layers
+//     and head at 17 / 32 / 48 / 64 rows 206 -> 185, 216 -> 196, 253 -> 224, 292 -> 262. Past 64 rows (two
+//     row blocks) single parts of 8 tiles stay: 70 us against 81 (10 tiles, two rounds).
+//   - otherwise 8 tiles; two parts where the grid is at most one round of workgroups and each has 8
+//     or more groups (Llama-3-8B at 64 rows: gate/up 47.5 -> 36.2 us, down); one where the grid
+//     already fills the CUs or the groups are few (QKV and o_proj split 5-8 ways over K; Qwen2-72B's
+//     gate/up at 32 rows, 462 workgroups: two parts 217 -> 226 us a layer).
 template <int EPI, int MT>
 hipError_t vx_pgemm_launch_t(const VxMMat& w, const VxBGemmArgs& a, hipStream_t st) {
     const uint32_t ks = a.ksplit > 1u ? a.ksplit : 1u;
-    const dim3 grid((w.n_tiles + kPTiles - 1u) / kPTiles, ks);
-    const uint64_t wgs = (uint64_t)grid.x * ks * ((a.batch + 16u * MT - 1u) / (16u * MT));
-    if (wgs <= 256u && w.n_grp / ks >= 8u) return vx_pgemm_launch_kh<EPI, MT, 2>(w, a, grid, st);
-    return vx_pgemm_launch_kh<EPI, MT, 1>(w, a, grid, st);
+    const uint32_t gx = vx_pgemm_grid(w.n_tiles), gz = (a.batch + 16u * MT - 1u) / (16u * MT);
+    if constexpr (EPI == VX_EPI_SWIGLU || EPI == VX_EPI_ARGMAX) {
+        const uint64_t small = (uint64_t)vx_mgemm_grid(w.n_tiles) * ((a.batch + 31u) / 32u);
+        if (small <= 512u && w.n_grp >= 4u) return vx_pgemm_launch_kh<EPI, 2, 4, 1>(w, a, st);
+    }
+    if constexpr (EPI == VX_EPI_SWIGLU) {
+        if (gx > 256u && (w.n_tiles + 9u) / 10u <= 256u && gz == 1u) return vx_pgemm_launch_kh<EPI, MT, 2, 5>(w, a, st);
+    }
+    if ((uint64_t)gx * ks * gz <= 256u && w.n_grp / ks >= 8u) return vx_pgemm_launch_kh<EPI, MT, 2, kMWaves>(w, a, st);
+    return vx_pgemm_launch_kh<EPI, MT, 1, kMWaves>(w, a, st);
 }
 
 template <int EPI, int MT>

@@ -313,10 +313,12 @@ def test_gemm_m_swiglu(hiplib, oracle, dev, F, H, batch, bm):
 
 
 @pytest.mark.parametrize("F,H,batch", [(16385, 608, 17), (20480, 608, 48), (20480, 416, 64), (20481, 608, 33), (8192, 416, 32),
-                                       (8193, 608, 32), (4090, 608, 50), (8192, 384, 20)])
+                                       (8193, 608, 32), (4090, 608, 50), (8192, 384, 20), (32768, 384, 20), (8201, 608, 65),
+                                       (16384, 384, 128), (20470, 608, 77), (32769, 384, 33), (40960, 96, 64), (40961, 96, 18)])
 def test_gemm_m_workgroup_shapes(hiplib, oracle, dev, F, H, batch):
     """Gate/up at the edges of the workgroup shapes: 10-tile workgroups from 2050 tiles to 2560, the two-tile ones
-    with K in four parts up to 512 workgroups and from 4 groups of K (parts of two groups and empty ones)."""
+    with K in four parts up to 512 workgroups and from 4 groups of K (parts of two groups and empty ones), 16- and
+    20-tile ones past a round of 8-tile workgroups, in one row block and two."""
     test_gemm_m_swiglu(hiplib, oracle, dev, F, H, batch, 1)
 
 

@@ -643,12 +643,16 @@ hipError_t vx_pgemm_launch_kh(const VxMMat& w, const VxBGemmArgs& a, hipStream_t
 //   - gate/up whose 8-tile workgroups are more than one round, at up to 64 rows, while 10-tile ones
 //     are not (2049-2560 tiles): 5 waves a part, two parts. Qwen2.5-7B's 2368 tiles left 40 of 256
 //     CUs with two workgroups and the others waiting for them: 33.7 -> 27.1 us at 32 rows; two layers
-//     and head at 17 / 32 / 48 / 64 rows 206 -> 185, 216 -> 196, 253 -> 224, 292 -> 262. Past 64 rows (two
-//     row blocks) single parts of 8 tiles stay: 70 us against 81 (10 tiles, two rounds).
+//     and head at 17 / 32 / 48 / 64 rows 206 -> 185, 216 -> 196, 253 -> 224, 292 -> 262.
+//   - gate/up past one round otherwise: 16-tile workgroups (8 waves, one part) where those are one round, else
+//     20-tile ones (10 waves). A CU's waves and its work stay the same or get fewer, and twice as many waves share
+//     each staged activation, which every workgroup reads from L2 again. At 128 rows (two row blocks):
+//     Llama-3-8B 448 -> 224 workgroups 60.1 -> 54.2 us, Qwen2.5-7B 592 -> 238 of 20 tiles 70.0 -> 64.1 (10 tiles and
+//     two parts, two rounds: 80.8); Qwen2-72B at 32 rows 462 -> 231 74.0 -> 70.7.
 //   - otherwise 8 tiles; two parts where the grid is at most one round of workgroups and each has 8
 //     or more groups (Llama-3-8B at 64 rows: gate/up 47.5 -> 36.2 us, down); one where the grid
 //     already fills the CUs or the groups are few (QKV and o_proj split 5-8 ways over K; Qwen2-72B's
-//     gate/up at 32 rows, 462 workgroups: two parts 217 -> 226 us a layer).
+//     462 gate/up workgroups at 32 rows: two parts 217 -> 226 us a layer).
 template <int EPI, int MT>
 hipError_t vx_pgemm_launch_t(const VxMMat& w, const VxBGemmArgs& a, hipStream_t st) {
     const uint32_t ks = a.ksplit > 1u ? a.ksplit : 1u;
@@ -658,7 +662,11 @@ hipError_t vx_pgemm_launch_t(const VxMMat& w, const VxBGemmArgs& a, hipStream_t 
         if (small <= 512u && w.n_grp >= 4u) return vx_pgemm_launch_kh<EPI, 2, 4, 1>(w, a, st);
     }
     if constexpr (EPI == VX_EPI_SWIGLU) {
-        if (gx > 256u && (w.n_tiles + 9u) / 10u <= 256u && gz == 1u) return vx_pgemm_launch_kh<EPI, MT, 2, 5>(w, a, st);
+        if (gx * gz > 256u) {
+            if (gz == 1u && (w.n_tiles + 9u) / 10u <= 256u) return vx_pgemm_launch_kh<EPI, MT, 2, 5>(w, a, st);
+            if ((w.n_tiles + 15u) / 16u * gz <= 256u) return vx_pgemm_launch_kh<EPI, MT, 1, 8>(w, a, st);
+            if ((w.n_tiles + 19u) / 20u * gz <= 256u) return vx_pgemm_launch_kh<EPI, MT, 1, 10>(w, a, st);
+        }
     }
     if ((uint64_t)gx * ks * gz <= 256u && w.n_grp / ks >= 8u) return vx_pgemm_launch_kh<EPI, MT, 2, kMWaves>(w, a, st);
     return vx_pgemm_launch_kh<EPI, MT, 1, kMWaves>(w, a, st);
@@ -677,12 +685,10 @@ hipError_t vx_mgemm_dispatch_mt(const VxMMat& w, const VxBGemmArgs& a, hipStream
     if (a.batch <= 16) return vx_mgemm_launch_t<EPI, 1>(w, a, st);  // (the LDS-shared kernel: B=8 3857 -> 3640 tok/s)
     if (a.batch <= 32) return vx_pgemm_launch_t<EPI, 2>(w, a, st);
     if (a.batch <= 48) return vx_pgemm_launch_t<EPI, 3>(w, a, st);
-    // 49-128 rows: blocks of 4 row tiles from the grid's z dimension. At 65-128 rows each weight
-    // tile is then read by two workgroups, but twice the workgroups (single K halves, two per CU)
-    // run out of phase with each other, so one's loads and barrier overlap the other's MFMAs: TTFT
-    // at 128 tokens 5.84-5.93 -> 5.70-5.78 ms (Llama-3-8B), 5.73-5.77 -> 5.49-5.55 ms (Qwen2.5-7B)
-    // against one block of 8 row tiles (two K halves per workgroup where one round of workgroups
-    // holds the grid), same box, three alternating runs each
+    // 49-128 rows: blocks of 4 row tiles from the grid's z dimension. At 65-128 rows each weight tile is
+    // then read by two workgroups (one block of 8 row tiles, registers for one activation set: TTFT at
+    // 128 tokens 5.84-5.93 against 5.70-5.78 ms of Llama-3-8B, 5.73-5.77 against 5.49-5.55 of Qwen2.5-7B, both
+    // with 8-tile workgroups)
     return vx_pgemm_launch_t<EPI, 4>(w, a, st);
 }
 

@@ -322,6 +322,13 @@ def test_gemm_m_workgroup_shapes(hiplib, oracle, dev, F, H, batch):
     test_gemm_m_swiglu(hiplib, oracle, dev, F, H, batch, 1)
 
 
+@pytest.mark.parametrize("n,k,batch,ks", [(6144, 640, 65, 5), (4608, 1024, 128, 7), (1030, 1024, 128, 8), (16390, 256, 100, 2),
+                                          (1024, 1024, 70, 8)])
+def test_gemm_m_split_store_past_64_rows(hiplib, oracle, dev, n, k, batch, ks):
+    """Split-K STORE over two row blocks on both sides of the 16-tile workgroups' range (129-256 workgroups)."""
+    test_gemm_m_store_and_residual(hiplib, oracle, dev, n, k, batch, ks, 1)
+
+
 def test_gemm_m_rejects_bad_arguments(hiplib, oracle, dev):
     blocks = _weights(oracle, 64, 576, 9)
     t = TiledQ4(hiplib, dev, blocks, 64, 576)

@@ -86,6 +86,19 @@ uint32_t vx_pgemm_ksplit(const VxMatPlan& m, uint32_t row_blocks) {
     return ks ? ks : 1u;
 }
 
+// K splits of QKV over more than 64 rows (two row blocks): as many as keep a grid of 16-tile workgroups within one
+// round, where that is more than half of it (the GEMM then takes those), else the rule above. More splits than
+// one round of 8-tile workgroups of two K parts takes, and half the activation reads (Llama-3-8B 2 -> 5, four
+// layers of a 128-token prompt 588 -> 580 us). A matrix that the rule above leaves whole stays whole.
+uint32_t vx_pgemm_ksplit_qkv_128(const VxMatPlan& m) {
+    const uint32_t ks8 = vx_pgemm_ksplit(m, 2u), wgs = (m.m_tiles + 15u) / 16u * 2u;
+    if (ks8 == 1u) return ks8;
+    uint32_t ks = 256u / wgs;
+    if (ks > 8u) ks = 8u;
+    if (ks > m.m_grp) ks = m.m_grp;
+    return wgs * ks > 128u ? ks : ks8;
+}
+
 }  // namespace
 
 struct VeloxHipModel {
@@ -120,9 +133,9 @@ struct VeloxHipModel {
     uint32_t ksplit_qkv_wide = 1;  // QKV over more than 16 rows
     uint32_t ksplit_o16 = 1, ksplit_down16 = 1;  // o_proj and down of up to 16 rows
     // over more than 64 rows, two 64-row blocks of workgroups: QKV, o_proj, down split less, so that one
-    // round holds both blocks and half the partials are written and folded (whole prefill step: Llama-3-8B at
-    // 128 rows QKV 5 -> 2 splits 642 -> 637 us, o_proj 8 -> 4 636, down 8 -> 4 638; Qwen2.5-7B at 1000 rows
-    // 7 -> 3, 8 -> 4, 8 -> 4: 2970 -> 2938, 2933, 2967)
+    // round holds both blocks and half the partials are written and folded (whole prefill step, each alone:
+    // Llama-3-8B at 128 rows o_proj 8 -> 4 642 -> 636 us, down 8 -> 4 638; Qwen2.5-7B at 1000 rows 2970 ->
+    // 2933, 2967); QKV on 16-tile workgroups where those fill the round
     uint32_t ksplit_qkv_128 = 1, ksplit_o_128 = 1, ksplit_down_128 = 1;
     // fp16 activation operands of the batched GEMMs (over the MFMA-layout copies): element k of row m
     // at m * x_ld + (k / 32) * x_bs + k % 32, block-major [k / 32][16-row-padded rows][32] (one operand
@@ -573,7 +586,7 @@ int velox_hip_model_create(const VeloxHipModelConfig* cfg, VeloxHipModel** out) 
         M->ksplit_o16 = vx_mgemm_ksplit16(M->layers[0].o);
         M->ksplit_down16 = vx_mgemm_ksplit16(M->layers[0].down);
         M->ksplit_qkv_wide = vx_pgemm_ksplit(M->layers[0].qkv, 1u);
-        M->ksplit_qkv_128 = vx_pgemm_ksplit(M->layers[0].qkv, 2u);
+        M->ksplit_qkv_128 = vx_pgemm_ksplit_qkv_128(M->layers[0].qkv);
         M->ksplit_o_128 = vx_pgemm_ksplit(M->layers[0].o, 2u);
         M->ksplit_down_128 = vx_pgemm_ksplit(M->layers[0].down, 2u);
         M->ksplit_o = vx_mgemm_ksplit(M->layers[0].o);

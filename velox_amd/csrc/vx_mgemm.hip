@@ -649,6 +649,10 @@ hipError_t vx_pgemm_launch_kh(const VxMMat& w, const VxBGemmArgs& a, hipStream_t
 //     each staged activation, which every workgroup reads from L2 again. At 128 rows (two row blocks):
 //     Llama-3-8B 448 -> 224 workgroups 60.1 -> 54.2 us, Qwen2.5-7B 592 -> 238 of 20 tiles 70.0 -> 64.1 (10 tiles and
 //     two parts, two rounds: 80.8); Qwen2-72B at 32 rows 462 -> 231 74.0 -> 70.7.
+//   - QKV split over K past 64 rows: 16-tile workgroups of one part where those fill more than half a round (the
+//     planner then splits to fill the round). Llama-3-8B, 5 splits for 2, two layers at 70 / 96 / 128 rows
+//     297 -> 292, 303 -> 300, 315 -> 312.9 us, Qwen2.5-7B within 0.3 %. o_proj and down stay (8 splits: Llama-3-8B
+//     315 -> 319, Qwen2.5-7B 337 -> 333).
 //   - otherwise 8 tiles; two parts where the grid is at most one round of workgroups and each has 8
 //     or more groups (Llama-3-8B at 64 rows: gate/up 47.5 -> 36.2 us, down); one where the grid
 //     already fills the CUs or the groups are few (QKV and o_proj split 5-8 ways over K; Qwen2-72B's
@@ -667,6 +671,10 @@ hipError_t vx_pgemm_launch_t(const VxMMat& w, const VxBGemmArgs& a, hipStream_t 
             if ((w.n_tiles + 15u) / 16u * gz <= 256u) return vx_pgemm_launch_kh<EPI, MT, 1, 8>(w, a, st);
             if ((w.n_tiles + 19u) / 20u * gz <= 256u) return vx_pgemm_launch_kh<EPI, MT, 1, 10>(w, a, st);
         }
+    }
+    if constexpr (EPI == VX_EPI_STORE) {
+        const uint64_t g16 = (uint64_t)((w.n_tiles + 15u) / 16u) * ks * gz;
+        if (ks > 1u && gz > 1u && g16 > 128u && g16 <= 256u) return vx_pgemm_launch_kh<EPI, MT, 1, 8>(w, a, st);
     }
     if ((uint64_t)gx * ks * gz <= 256u && w.n_grp / ks >= 8u) return vx_pgemm_launch_kh<EPI, MT, 2, kMWaves>(w, a, st);
     return vx_pgemm_launch_kh<EPI, MT, 1, kMWaves>(w, a, st);

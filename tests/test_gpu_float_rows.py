@@ -189,7 +189,7 @@ def test_runner_unquantized_fp32_matches_the_engine(oracle):
 @pytest.mark.parametrize("ffn", [16384, 29568])
 def test_wide_rows_past_64k_of_lds(oracle, quant, ffn):
     """The float-row GEMV holds a row's fp32 activations in LDS: the down projection's 16384-wide rows
-    take 65,600 bytes and Qwen2-72B's 29568-wide ones 118,336, past the 64 KiB default the launch
+    take 65,632 bytes and Qwen2-72B's 29568-wide ones 118,368, past the 64 KiB default the launch
     raises. One layer of that width decodes within the fp32-accumulation bar of the oracle on the
     GPU's own K/V rows."""
     cfg = dict(vocab_size=512, hidden_dim=256, intermediate_dim=ffn, num_layers=1, num_heads=4, num_kv_heads=2,
@@ -235,3 +235,38 @@ def test_float_rows_grid_edges_match_the_oracle(oracle, quant, hidden, inter, he
         assert tg == oracle.argmax(gpu.logits) and err < F32_TOL, (pos, err)
     gpu.close()
     ref.close()
+
+
+def _load_model(gpu, cfg, quant, tensors, gains):
+    """Every matrix of a small model (zeros unless given) and its gains (1 unless given) through the row loaders."""
+    h, f, v = cfg["hidden_dim"], cfg["intermediate_dim"], cfg["vocab_size"]
+    qd, kvd = cfg["num_heads"] * cfg["head_dim"], cfg["num_kv_heads"] * cfg["head_dim"]
+    shapes = {L.T_EMBED: (v, h), L.T_Q: (qd, h), L.T_K: (kvd, h), L.T_V: (kvd, h), L.T_O: (h, qd), L.T_GATE: (f, h),
+              L.T_UP: (f, h), L.T_DOWN: (h, f)}
+    for kind, shape in shapes.items():
+        x = np.ascontiguousarray(tensors.get(kind, np.zeros(shape)), np.float16 if quant == L.QUANT_F16 else np.float32)
+        L.check(gpu.lib.velox_hip_load_rows(C.byref(gpu.arena), kind, 0, x.ctypes.data, x.nbytes, None), kind)
+    for kind in (L.T_ATTN_NORM, L.T_MLP_NORM, L.T_FINAL_NORM):
+        gpu.load_f32(kind, 0, gains.get(kind, np.ones(h, np.float32)))
+
+
+TINY = dict(vocab_size=33, hidden_dim=64, intermediate_dim=96, num_layers=1, num_heads=1, num_kv_heads=1, head_dim=64,
+            rms_norm_eps=1e-5, rope_theta=10000.0, qkv_bias=0, tied_lm_head=1)
+
+
+@pytest.mark.parametrize("quant", [L.QUANT_F32, L.QUANT_F16])
+def test_infinite_last_activation_of_a_ragged_row(quant):
+    """An infinite activation in the last 16-byte word of rows that are no multiple of a wave's 64 words (24 or
+    12 here): gate and up are 0 but for their last row, whose product overflows, so each hidden value is
+    infinity with the sign of its down weight. Lanes past the row's end add nothing (0 times it is no number)."""
+    rng = np.random.default_rng(3)
+    e = rng.choice([-1.0, 1.0], 64) * rng.uniform(0.5, 1.0, 64)
+    last = np.zeros((96, 64))
+    last[95] = e
+    down = rng.choice([-1.0, 1.0], (64, 96)) * rng.uniform(0.01, 0.05, (64, 96))
+    gpu = HipDecodeEngine(dict(TINY, quant_mode=quant), max_seq_len=4, synthesize=False)
+    _load_model(gpu, TINY, quant, {L.T_EMBED: np.tile(e, (33, 1)), L.T_GATE: last, L.T_UP: last, L.T_DOWN: down},
+                {L.T_MLP_NORM: np.full(64, 1e20, np.float32)})
+    gpu.forward_step(5, 0)
+    assert np.array_equal(gpu.read_hidden(), np.copysign(np.inf, down[:, 95]).astype(np.float32))
+    gpu.close()

@@ -24,6 +24,8 @@
 namespace {
 
 constexpr int kFWaves = 8, kFThreads = 64 * kFWaves;  // at most; the launcher picks 1..8 waves
+constexpr uint32_t kFPad = 8;                          // zeros after the row's activations: one word's worth
+constexpr uint32_t vf_lds(uint32_t k) { return (k + kFPad + 2u * kFWaves) * 4u; }
 
 typedef uint32_t vf_u4 __attribute__((ext_vector_type(4)));
 typedef float vf_f4 __attribute__((ext_vector_type(4)));
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(kFThreads) void vx_gemv_f_kernel(VxMat m, VxGemvArg
     constexpr int GX = SPL > 0 ? 1 : NORM ? 2 : 4;  // float4 of x per thread requested before the weights
     const uint32_t K = m.k, K4 = K / 4u;
     float* xs = vf_smem;
-    float* red = vf_smem + K;  // [kFWaves] partial sums, then the argmax candidates
+    float* red = vf_smem + K + kFPad;  // [kFWaves] partial sums, then the argmax candidates
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t nwv = blockDim.x >> 6, nth = blockDim.x;
 
@@ -174,6 +176,7 @@ __global__ __launch_bounds__(kFThreads) void vx_gemv_f_kernel(VxMat m, VxGemvArg
         load_x(0, i);
         stage(0, i);
     }
+    if (tid < (int)kFPad) xs[K + tid] = 0.0f;
     if constexpr (NORM) {
         ss = vf_wave_sum(ss);
         if (lane == 0) red[wave] = ss;
@@ -195,8 +198,8 @@ __global__ __launch_bounds__(kFThreads) void vx_gemv_f_kernel(VxMat m, VxGemvArg
     uint32_t ci = 0, j = r0;  // current item
     auto consume = [&](int u) {
         const uint32_t c = ci * 64u + (uint32_t)lane;
-        const bool in = c < nw;  // past the row's end: zero weights
-        const float* x = xs + min(c, nw - 1u) * E;
+        const bool in = c < nw;  // past the row's end: zero weights, and the zeros after xs (0 times infinity is no 0)
+        const float* x = xs + min(c, nw) * E;
 #pragma unroll
         for (int p = 0; p < PR; ++p) {
             vf_u4 q = w[u][p];
@@ -286,14 +289,14 @@ void vf_grid(uint32_t n, int epi, uint32_t head_wgs, uint32_t max_wgs, uint32_t&
 
 template <typename T, int EPI, bool NORM, int SPL>
 hipError_t vx_gemv_f_launch_t(const VxMat& m, const VxGemvArgs& a, dim3 grid, hipStream_t st) {
-    const size_t lds = (size_t)m.k * 4u + 2u * kFWaves * 4u;
-    // rows wider than 16376 need more than the default 64 KiB of dynamic LDS (up to 128 KiB + 64 B
+    const size_t lds = vf_lds(m.k);
+    // rows wider than 16360 need more than the default 64 KiB of dynamic LDS (up to 128 KiB + 96 B
     // at kVxFloatMaxK, of the 160 KiB a CU has): raised once per instantiation to the widest row
     static bool attr_set = false;
     if (lds > 65536u && !attr_set) {
         if (hipFuncSetAttribute((const void*)vx_gemv_f_kernel<T, EPI, NORM, SPL>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)((size_t)kVxFloatMaxK * 4u + 2u * kFWaves * 4u)) != hipSuccess) {
+                                (int)vf_lds(kVxFloatMaxK)) != hipSuccess) {
             (void)hipGetLastError();
             return hipErrorInvalidValue;
         }

@@ -270,3 +270,21 @@ def test_infinite_last_activation_of_a_ragged_row(quant):
     gpu.forward_step(5, 0)
     assert np.array_equal(gpu.read_hidden(), np.copysign(np.inf, down[:, 95]).astype(np.float32))
     gpu.close()
+
+
+@pytest.mark.parametrize("gain", [1.0, 2.0])
+def test_rmsnorm_of_values_whose_squares_overflow(gain):
+    """Activations of 3e38: their mean square is infinite and 1 / rms is 0, so every normalized value, and with it
+    every projection, is 0 (x * gain, or a product of it, that overflows before 1 / rms reaches it is not)."""
+    rng = np.random.default_rng(4)
+    e = (rng.choice([-1.0, 1.0], 64) * rng.uniform(2.9e38, 3.3e38, 64)).astype(np.float32)
+    w = {kind: rng.normal(0, 2, shape) for kind, shape in (
+        (L.T_Q, (64, 64)), (L.T_K, (64, 64)), (L.T_V, (64, 64)), (L.T_O, (64, 64)), (L.T_GATE, (96, 64)),
+        (L.T_UP, (96, 64)), (L.T_DOWN, (64, 96)))}
+    gpu = HipDecodeEngine(dict(TINY, quant_mode=L.QUANT_F32), max_seq_len=4, synthesize=False)
+    g = np.full(64, gain, np.float32)
+    _load_model(gpu, TINY, L.QUANT_F32, {L.T_EMBED: np.tile(e, (33, 1)), **w},
+                {L.T_ATTN_NORM: g, L.T_MLP_NORM: g, L.T_FINAL_NORM: g})
+    gpu.forward_step(5, 0)
+    assert np.array_equal(gpu.read_hidden(), e) and not gpu.logits.any()
+    gpu.close()

@@ -187,6 +187,15 @@ __global__ __launch_bounds__(kFThreads) void vx_gemv_f_kernel(VxMat m, VxGemvArg
         float tot = 0.0f;
         for (uint32_t v = 0; v < nwv; ++v) tot += red[v];
         inv_rms = 1.0f / sqrtf(tot / (float)K + a.eps);
+        if (!(tot < 1e30f)) {  // (workgroup-uniform) x may pass 1e15: 1 / rms goes first, or the sums overflow before it
+            for (uint32_t i = (uint32_t)tid; i < K4; i += nth) {
+                const float4 v = ((const float4*)a.x)[i], g = ((const float4*)a.gain)[i];
+                ((float4*)xs)[i] = make_float4((v.x * inv_rms) * g.x, (v.y * inv_rms) * g.y, (v.z * inv_rms) * g.z,
+                                               (v.w * inv_rms) * g.w);
+            }
+            inv_rms = 1.0f;
+            __syncthreads();
+        }
     }
 
     // ---- stream: consume item u, refill it with the item U ahead, finish rows on the fly ----

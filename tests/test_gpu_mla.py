@@ -179,7 +179,9 @@ def test_mla_bad_arguments():
 @pytest.mark.parametrize("heads,batch,splits,max_seq", [
     (64, 16, 16, 96),    # splits of one 32-position chunk, most of them empty
     (64, 32, 8, 1300),   # splits of up to six chunks, sequences ending anywhere in them
-    (128, 5, 28, 700),   # two head groups, 280 workgroups dealt unevenly to the eight XCDs
+    (128, 5, 28, 700),   # two head groups, 280 workgroups: past one per CU, 10 (sequence, group) runs for 8 XCDs
+    (64, 19, 14, 1300),  # 266 workgroups of unequal length, 19 sequences for 8 XCDs
+    (128, 9, 14, 440),   # 252 workgroups, dealt unevenly to the eight XCDs
 ])
 def test_mla_attention_64_heads_vs_oracle(oracle, heads, batch, splits, max_seq):
     """The 64-head attention workgroups at the edges of chunks and splits: contexts of 0 positions, one

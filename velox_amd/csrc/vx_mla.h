@@ -59,6 +59,27 @@ struct VxMlaAttnArgs {
     uint64_t active_mask;
 };
 
+// What workgroup `block` of the 64-head attention's grid takes: split, sequence and group of 64 heads, of
+// `groups` head groups (sp = splits: nothing). The dispatcher deals workgroup i to XCD i % 8.
+// - Up to one workgroup per CU, XCD x takes items [x share, (x + 1) share) in the order (sequence, split, head
+//   group), so a split's head groups read its latent rows, and a sequence's splits its q, through one L2 (q
+//   through all eight cost about 4 us of a launch).
+// - Past that a CU takes a second item when its first is done, and sequences are of unequal length: the first
+//   splits of every sequence come first, dealt to every XCD in turn, the last ones, empty for the shorter
+//   sequences, last. In the order above the XCD of the longest sequences ran a second round alone. One
+//   DeepSeek-V3 layer, lengths from 3400 down to half: 13 sequences 129.3 -> 110.3 us, 20 171.9 -> 153.5,
+//   24 190.9 -> 164.5, 31 207.6 -> 184.3 (of equal length: 12 123.7 -> 127.5, 19 172.1 and 172.4, 26 198.6 -> 196.8).
+struct VxMlaItem {
+    uint32_t sp, b, hg;
+};
+__host__ __device__ inline VxMlaItem vx_mla_attn64_item(uint32_t block, uint32_t splits, uint32_t batch, uint32_t groups) {
+    const uint32_t runs = batch * groups, items = splits * runs;
+    if (items > 256u) return {block / runs, block % runs / groups, block % groups};
+    const uint32_t share = (items + 7u) / 8u, item = (block & 7u) * share + (block >> 3);
+    if (item >= items) return {splits, 0u, 0u};  // the grid is rounded up to whole shares
+    return {item / groups % splits, item / (groups * splits), item % groups};
+}
+
 hipError_t vx_launch_f8_synth_scales(float* scales, uint32_t rows, uint32_t cols, uint64_t stream, float coef,
                                      hipStream_t st);
 hipError_t vx_launch_f8_pack(const VxF8Dest& d, hipStream_t st);

@@ -1062,7 +1062,7 @@ __global__ __launch_bounds__(64 * W * LS, 1) void vx_mla_attn_kernel(VxMlaAttnAr
 // * P.V: wave w accumulates all 64 heads over LR / 8 dimensions, so each latent value is read once per
 //   workgroup (P, 4 KiB, once per wave);
 // * P.V of chunk i runs in the phase of the scores of chunk i + 1: two barriers per chunk.
-// * O leaves through LDS as whole lines, and a sequence's workgroups share an XCD (below).
+// * O leaves through LDS as whole lines; within one round a sequence's workgroups share an XCD (vx_mla_attn64_item).
 // DeepSeek-V3 at B = 16, 8 splits of 17 chunks: 47.4 -> 36.0 us (kernel trace); what is left is about 13 us
 // before the first chunk and after the last (q, the partials' 16.8 MB) and 1.4 us per chunk, of which
 // barriers and softmax 0.5, the scores' LDS reads 0.3, P.V 0.3, the loads 0.2 (by elimination).
@@ -1106,13 +1106,9 @@ __global__ __launch_bounds__(512) void vx_mla_attn64_kernel(VxMlaAttnArgs a, uin
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hm = wave >> 1, pb = wave & 1;
     const int col = lane & 15, grp = lane >> 4;
-    // The dispatcher deals workgroup i to XCD i % 8: XCD x takes items [x share, (x + 1) share) in the order
-    // (sequence, split, head group), so a split's head groups read its latent rows, and a sequence's splits
-    // its q, through one L2 (q through all eight cost about 4 us of a launch).
-    const uint32_t zg = a.nh / 64u, items = batch * a.splits * zg, share = gridDim.x / 8u;
-    const uint32_t item = (blockIdx.x & 7u) * share + (blockIdx.x >> 3);
-    if (item >= items) return;  // the grid is rounded up to whole shares
-    const uint32_t sp = item / zg % a.splits, b = item / (zg * a.splits), hbase = item % zg * 64u;
+    const VxMlaItem it = vx_mla_attn64_item(blockIdx.x, a.splits, batch, a.nh / 64u);
+    if (it.sp >= a.splits) return;
+    const uint32_t sp = it.sp, b = it.b, hbase = it.hg * 64u;
     const uint32_t head = hbase + 16u * (uint32_t)hm + (uint32_t)col;
     const uint64_t step = a.states[b].step;
     const uint32_t pos = __builtin_amdgcn_readfirstlane(step < (uint64_t)a.s_max ? (uint32_t)step : a.s_max - 1u);
@@ -1464,6 +1460,14 @@ hipError_t vx_mla_attn_launch_t(const VxMlaAttnArgs& a, uint32_t batch, hipStrea
     hipLaunchKernelGGL((vx_mla_attn_kernel<LR, DR, W, LS>), dim3(a.splits, batch, a.nh / (16u * W)),
                        dim3(64 * W * LS), lds, st, a);
     return hipGetLastError();
+}
+
+// (vx_mla_attn64_item for the CPU test of the dealing)
+extern "C" void vx_mla_attn64_deal(uint32_t block, uint32_t splits, uint32_t batch, uint32_t groups, uint32_t* out) {
+    const VxMlaItem it = vx_mla_attn64_item(block, splits, batch, groups);
+    out[0] = it.sp;
+    out[1] = it.b;
+    out[2] = it.hg;
 }
 
 hipError_t vx_mla_attn64_launch(const VxMlaAttnArgs& a, uint32_t batch, hipStream_t st) {

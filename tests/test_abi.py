@@ -185,6 +185,23 @@ def test_tiled_layout_choices():
     assert lib.velox_hip_q4_layout(10, 64, 64, 1, C.byref(m), None, None) == -1
 
 
+@pytest.mark.parametrize("n,k,want", [
+    (576, 576, (192, 3)), (1536, 576, (256, 6)), (64, 96, (64, 1)), (2048, 29568, (256, 8)),
+    (4096, 14336, (512, 8)),    # 57 KB of activations: two workgroups a CU
+    (3584, 18944, (448, 8)), (8192, 8192, (1024, 8)),
+    (8192, 29568, (256, 8)),    # 118 KB: one workgroup a CU, 1024 would be four rounds
+    (2304, 20456, (288, 8)), (2304, 20480, (256, 8)),  # the last width of two a CU and the next
+    (8192, 16384, (256, 8)), (8193, 576, (256, 8)), (28672, 4096, (256, 8)),
+])
+def test_float_row_grid(n, k, want):
+    """Workgroups and waves of the float-row GEMV: one row per wave while that is one round, else max_wgs (256)."""
+    wgs, waves = C.c_uint32(), C.c_uint32()
+    L.load().vx_gemv_f_grid(n, k, 0, 99, 256, C.byref(wgs), C.byref(waves))
+    assert (wgs.value, waves.value) == want
+    L.load().vx_gemv_f_grid(n, k, 3, 99, 256, C.byref(wgs), C.byref(waves))  # the LM head: the caller's
+    assert (wgs.value, waves.value) == (99, 8)
+
+
 def test_bench_refuses_multi_gpu():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True,
                        timeout=60)

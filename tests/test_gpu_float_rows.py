@@ -215,6 +215,7 @@ def test_wide_rows_past_64k_of_lds(oracle, quant, ffn):
     (64, 96, 1, 1, 64, 33),         # rows shorter than a wave's 64 words, 1-wave workgroups, fewer rows than CUs
     (264 * 4, 1536, 9, 3, 64, 301),  # a ragged last word group (264 / 132 words), 6-wave workgroups
     (2080, 4160, 16, 4, 128, 2055),  # 8-wave workgroups: several rows per wave, uneven blocks of rows
+    (2080, 20480, 2, 1, 128, 33),    # rows too wide for two workgroups a CU: 260 workgroups become 256
 ])
 def test_float_rows_grid_edges_match_the_oracle(oracle, quant, hidden, inter, heads, kv, d, vocab):
     """The float-row GEMV's grids and row ends: two layers, three positions, within the fp32-accumulation bar."""

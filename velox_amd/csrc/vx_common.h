@@ -341,8 +341,8 @@ int vx_record_error(hipError_t e);  // vx_host.cpp: the first error of a step, r
 enum { VX_EPI_STORE = 0, VX_EPI_RESID = 1, VX_EPI_SWIGLU = 2, VX_EPI_ARGMAX = 3 };
 hipError_t vx_launch_gemv(const VxMat& m, const VxGemvArgs& a, int epi, uint32_t max_wgs, hipStream_t st);
 // The float-row GEMV (vx_gemv_f.hip) that vx_launch_gemv runs for VX_FMT_F32 / VX_FMT_F16 matrices,
-// its grid from the rows (past 8192 rows at most max_wgs workgroups; the LM head: head_wgs, vx_gemv_grid
-// of the matrix's tiles).
+// its grid from the rows (past 8192 rows, or past one round of what a CU's LDS holds, at most max_wgs
+// workgroups; the LM head: head_wgs, vx_gemv_grid of the matrix's tiles).
 hipError_t vx_launch_gemv_f(const VxMat& m, const VxGemvArgs& a, int epi, uint32_t head_wgs, uint32_t max_wgs,
                             hipStream_t st);
 hipError_t vx_launch_attention(const VxAttnArgs& a, uint32_t d, hipStream_t st);

@@ -13,7 +13,7 @@
 //
 // What bounds it: HBM for wide matrices, the first bytes' latency for SmolLM's (0.3-7 MB a launch).
 // Both want every CU to hold loads from the start: one row per wave puts SmolLM's 576-1536 rows on
-// 192-256 workgroups (tiles of 4 rows filled 18-48), each wave's first kFRing words are requested
+// 192-256 workgroups (tiles of 4 rows filled 18-48), each wave's first U words are requested
 // before the input is staged (they arrive while it is), and the ring of words in flight runs on over
 // row ends.
 #include <hip/hip_fp16.h>
@@ -277,24 +277,34 @@ __global__ __launch_bounds__(kFThreads) void vx_gemv_f_kernel(VxMat m, VxGemvArg
     }
 }
 
+}  // namespace
+
 // Grid: 1..8 waves per workgroup so that up to 2048 rows, one per wave, make at most 256 workgroups
-// (SmolLM's 576-1536 rows: 192-256); up to 8192 rows one row per wave in 8-wave workgroups (a wave's
-// whole row is then requested at once: Llama-3-8B's 4096-row down projection in fp16 20.6 us on 512
-// workgroups, 21.0 with max_wgs = 256); more rows max_wgs workgroups, each wave streaming several rows
-// (its gate/up, 28672 rows: 36.1 us, 6.5 TB/s). The LM head's grid is the caller's (its finalize
+// (SmolLM's 576-1536 rows: 192-256); up to 8192 rows one row per wave in 8-wave workgroups (the wave's
+// first U words of its row, all of a short one, are then requested at once: Llama-3-8B's 4096-row down
+// projection in fp16 20.6 us on 512 workgroups, 21.0 with max_wgs = 256), where a CU's LDS and 32 waves hold
+// them all in one round; otherwise, and for more rows, max_wgs workgroups, each wave streaming several rows
+// (Llama-3-8B's gate/up, 28672 rows: 36.1 us, 6.5 TB/s; Qwen2-72B's down, 8192 rows of 29568 in 118 KB of LDS:
+// four rounds of 256 workgroups, each staging the activations again, 83.7 us, one 80.0; its o_proj, 8192 rows of
+// 8192, is one round of 1024, 27.8 us, 27.3 on 256). The LM head's grid is the caller's (its finalize
 // kernel reads one candidate per workgroup). Against tiles of 4 rows per wave, kernel trace: SmolLM
 // fp32 gate/up 7.0 -> 3.2 us, down 6.9 -> 2.8, QKV 5.2 -> 2.9, o_proj 5.4 -> 3.2; Llama-3-8B fp16
-// gate/up 43.8 -> 36.1, down 28.7 -> 20.6, QKV 14.2 -> 10.6, o_proj 11.6 -> 9.0 us.
-void vf_grid(uint32_t n, int epi, uint32_t head_wgs, uint32_t max_wgs, uint32_t& wgs, uint32_t& waves) {
-    waves = min((n + 255u) / 256u, (uint32_t)kFWaves);
+// gate/up 43.8 -> 36.1, down 28.7 -> 20.6, QKV 14.2 -> 10.6, o_proj 11.6 -> 9.0 us; Qwen2-72B fp16 o_proj
+// 32.6 -> 27.8, down 81.0 -> 80.0.
+extern "C" void vx_gemv_f_grid(uint32_t n, uint32_t k, int epi, uint32_t head_wgs, uint32_t max_wgs, uint32_t* wgs,
+                               uint32_t* waves) {
+    *waves = min((n + 255u) / 256u, (uint32_t)kFWaves);
     if (epi == VX_EPI_ARGMAX) {
-        waves = kFWaves;
-        wgs = head_wgs;
+        *waves = kFWaves;
+        *wgs = head_wgs;
         return;
     }
-    wgs = (n + waves - 1u) / waves;
-    if (n > 8192u) wgs = min(wgs, max_wgs ? max_wgs : 1u);
+    *wgs = (n + *waves - 1u) / *waves;
+    const uint32_t per_cu = min(160u * 1024u / vf_lds(k), 4u);
+    if (n > 8192u || *wgs > 256u * per_cu) *wgs = min(*wgs, max_wgs ? max_wgs : 1u);
 }
+
+namespace {
 
 template <typename T, int EPI, bool NORM, int SPL>
 hipError_t vx_gemv_f_launch_t(const VxMat& m, const VxGemvArgs& a, dim3 grid, hipStream_t st) {
@@ -354,7 +364,7 @@ hipError_t vx_launch_gemv_f(const VxMat& m, const VxGemvArgs& a, int epi, uint32
     if ((epi == VX_EPI_SWIGLU) != (m.paired != 0)) return hipErrorInvalidValue;
     if (epi == VX_EPI_ARGMAX && (!a.cand_v || !a.cand_i)) return hipErrorInvalidValue;
     uint32_t wgs, waves;
-    vf_grid(m.n, epi, head_wgs, max_wgs, wgs, waves);
+    vx_gemv_f_grid(m.n, m.k, epi, head_wgs, max_wgs, &wgs, &waves);
     const dim3 grid(wgs, waves);  // (workgroups, waves per workgroup)
     if (m.fmt == VX_FMT_F32) return vx_gemv_f_epi<float>(m, a, epi, grid, st);
     if (m.fmt == VX_FMT_F16) return vx_gemv_f_epi<__half>(m, a, epi, grid, st);

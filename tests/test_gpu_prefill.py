@@ -308,3 +308,12 @@ def test_prefill_row_blocks_and_long_contexts_vs_oracle(oracle, chunk, rows):
     cfg = dict(vocab_size=512, hidden_dim=384, intermediate_dim=640, num_heads=14, num_kv_heads=2, head_dim=128,
                rms_norm_eps=1e-6, rope_theta=1000000.0, qkv_bias=1, tied_lm_head=1)
     _prefill_vs_oracle(oracle, cfg, 2, chunk, rows, [(0, rows)], rows + 20, seed=83, decode_steps=1)
+
+
+@pytest.mark.parametrize("chunk,rows,bias", [(16, 23, 1), (128, 150, 1), (128, 101, 0)])
+def test_prefill_of_unsplit_qkv_vs_oracle(oracle, chunk, rows, bias):
+    """QKV rows too many to split over K (10240: Qwen2-72B's, 64 q heads over 8 KV heads) in chunks of up to 16 and
+    past 64 rows: the whole rows are the one partial of the attention's 2-row workgroups, with and without a bias."""
+    cfg = dict(vocab_size=512, hidden_dim=256, intermediate_dim=384, num_heads=64, num_kv_heads=8, head_dim=128,
+               rms_norm_eps=1e-6, rope_theta=1000000.0, qkv_bias=bias, tied_lm_head=1)
+    _prefill_vs_oracle(oracle, cfg, 2, chunk, rows, [(0, rows)], rows + 20, seed=84, decode_steps=1)

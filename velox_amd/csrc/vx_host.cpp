@@ -1233,15 +1233,19 @@ void vx_rows_forward(const VeloxHipModel* M, VeloxHipArena* A, const VeloxDecode
             g.pstride = (uint64_t)M->rows * g.ldy;
         }
         vx_record(gemm(L.qkv, g, VX_EPI_STORE));
-        // QKV split over K: the K/V-row and attention kernels sum the partials (+ bias) themselves
-        at.qkv_nparts = g.ksplit > 1 ? g.ksplit : 0u;
-        at.qkv_part = part_r;
-        at.qkv_pstride = g.pstride;
-        at.qkv_bias = g.bias;
+        // QKV split over K: the K/V-row and attention kernels sum the partials (+ bias) themselves. Whole QKV rows
+        // (bias added) are the one partial of a prefill chunk of more than 16 rows: its attention then takes 16 / G
+        // rows per workgroup. One Qwen2-72B layer, 10240 QKV rows: 100 rows at 7000 positions 708 us with one row
+        // per workgroup, 566 with two; 65 at 2000 475 and 456; 16 at 2000 196.5 and 199.5, 2 at 0 162.5 and 166.6.
+        const bool split = g.ksplit > 1;
+        at.qkv_nparts = split ? g.ksplit : prefill && n > 16u ? 1u : 0u;
+        at.qkv_part = split ? part_r : qkv;
+        at.qkv_pstride = split ? g.pstride : 0;
+        at.qkv_bias = split ? g.bias : nullptr;
         at.kv = vx_kv(M, A, l, 0);
         if (prefill)
-            vx_record(vx_launch_kv_append_rows(at.qkv_nparts ? part_r : qkv, qd + 2 * kvd, at.qkv_nparts, g.pstride,
-                                               g.bias, c.num_heads, c.num_kv_heads, D, rows, n, at.rope,
+            vx_record(vx_launch_kv_append_rows(at.qkv_part, qd + 2 * kvd, split ? g.ksplit : 0u, at.qkv_pstride,
+                                               at.qkv_bias, c.num_heads, c.num_kv_heads, D, rows, n, at.rope,
                                                c.max_seq_len, M->s_cap, at.kv, mask, st));
         vx_record(vx_launch_attention(at, D, st));
         if (bsplits > 1)  // (one split: the attention wrote the o_proj operand itself)

@@ -743,9 +743,11 @@ hipError_t vx_attn_launch_w(const VxAttnArgs& a, hipStream_t st) {
 template <int D, int G, bool PS>
 hipError_t vx_attn_launch_ps(const VxAttnArgs& a, hipStream_t st) {
     if constexpr (PS) {
-        // prefill chunks: 16 / G rows per workgroup; 4 waves while they take every 32-position chunk in one
-        // pass, 8 beyond (a 128-row chunk is about one workgroup per CU: at 129-1000 positions of Qwen2.5-7B
-        // 18.3 -> 15.7 us median, 23.3 -> 20.0 in the last chunk)
+        // prefill chunks: 16 / G rows per workgroup, of 8 waves past 128 positions (a 128-row chunk is about one
+        // workgroup per CU: at 129-1000 positions of Qwen2.5-7B 18.3 -> 15.7 us median, 23.3 -> 20.0 in the last
+        // chunk). By the rows' positions, not by those of a split: a short tail's splits of up to 128 positions leave
+        // 4 of the 8 waves without a chunk, but the rows' q staging is the longer part (10 rows at 200 positions, two
+        // splits: Qwen2.5-7B 13.4 us with 4 waves, 10.8 with 8, Llama-3-8B 11.3 and 9.7, SmolLM 7.4 and 6.7)
         constexpr int R = 16 / G;
         if constexpr (R > 1)
             if (a.prefill)

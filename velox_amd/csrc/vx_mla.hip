@@ -1075,7 +1075,7 @@ __device__ __forceinline__ void vm_barrier() { asm volatile("s_waitcnt lgkmcnt(0
 
 // 16 bytes per lane from base + off (off per lane) to the 1 KiB of LDS at byte offset lds (both uniform)
 __device__ __forceinline__ void vm_dma16(const void* base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
 
 // The maximum over the four 16-lane groups, in every lane (lane swaps: no LDS round trip).

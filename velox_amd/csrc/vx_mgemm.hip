@@ -672,7 +672,7 @@ hipError_t vx_pgemm_launch_t(const VxMMat& w, const VxBGemmArgs& a, hipStream_t 
             if ((w.n_tiles + 19u) / 20u * gz <= 256u) return vx_pgemm_launch_kh<EPI, MT, 1, 10>(w, a, st);
         }
     }
-    if constexpr (EPI == VX_EPI_STORE) {
+    if constexpr (EPI == VX_EPI_STORE && MT == 4) {  // (two row blocks: more than 64 rows)
         const uint64_t g16 = (uint64_t)((w.n_tiles + 15u) / 16u) * ks * gz;
         if (ks > 1u && gz > 1u && g16 > 128u && g16 <= 256u) return vx_pgemm_launch_kh<EPI, MT, 1, 8>(w, a, st);
     }

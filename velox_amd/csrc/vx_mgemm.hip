@@ -406,7 +406,9 @@ __global__ __launch_bounds__(64 * PW * KH) void vx_pgemm_kernel(VxMMat w, VxBGem
     // i + 1 + XS. Every set index is a compile-time constant (the loop is unrolled by the ring size).
     vx_mu4 cw[kPRing][NT];
     vx_mu2 sw[kPRing][NT];
-    constexpr int XS = MT <= 4 ? 2 : 1;  // activation register sets (one at 8 row tiles: registers)
+    // activation register sets: one where 10 waves (168 registers each) stage 4 units a wave; two spilled 8 registers
+    // (Qwen2.5-7B gate/up at 64 rows 41.3 -> 36.9 us)
+    constexpr int XS = KH * PW > 8 && UPW > 3 ? 1 : 2;
     vx_mh8 xr[XS][UPW];
     auto load_w = [&](auto pc, uint32_t j) {
         constexpr int p = decltype(pc)::value;
